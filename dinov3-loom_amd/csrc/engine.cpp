@@ -190,7 +190,8 @@ void validate(const dhx_engine* e, const dhx_launch& l) {
     }
 }
 
-hipError_t launch_one(dhx_engine* e, const dhx_launch& l, hipStream_t stream) {
+// shared: launches of other branches run beside this one.
+hipError_t launch_one(dhx_engine* e, const dhx_launch& l, hipStream_t stream, bool shared) {
     using namespace dhx;
     auto P = [&](int i) { return region_ptr(e, l.bindings[i]); };
     auto F = [&](int i) { return static_cast<const float*>(P(i)); };
@@ -215,9 +216,9 @@ hipError_t launch_one(dhx_engine* e, const dhx_launch& l, hipStream_t stream) {
         case DHX_K_ATTENTION:
             return launch_attention({Hf(0), Hf(1), Hf(2), Hf(3), (int)s[0], (int)tokens_for(s[1]), (int)s[2]}, stream);
         case DHX_K_RESID:
-            return launch_resid({Hf(0), Hf(1), F(2), F(3), Hf(4), (int)s[0], (int)s[1]}, stream);
+            return launch_resid({Hf(0), Hf(1), F(2), F(3), Hf(4), (int)s[0], (int)s[1], nullptr, shared}, stream);
         case DHX_K_RESID_STATS:
-            return launch_resid({Hf(0), Hf(1), F(2), F(3), Hf(4), (int)s[0], (int)s[1], Fm(5)}, stream);
+            return launch_resid({Hf(0), Hf(1), F(2), F(3), Hf(4), (int)s[0], (int)s[1], Fm(5), shared}, stream);
         case DHX_K_SWIGLU:
             return launch_swiglu({Hf(0), Hf(1), F(2), Hf(3), (int)s[0]}, stream);
         case DHX_K_SWIGLU_LN:
@@ -265,7 +266,8 @@ hipError_t queue_branches(dhx_engine* e, const Recorded& r) {
     size_t first = 0;
     for (size_t i = 0; i < n; ++i) {
         hipStream_t s = i == 0 ? e->stream : e->aux[i - 1];
-        for (size_t j = first; j < first + r.counts[i] && err == hipSuccess; ++j) keep(launch_one(e, r.launches[j], s));
+        for (size_t j = first; j < first + r.counts[i] && err == hipSuccess; ++j)
+            keep(launch_one(e, r.launches[j], s, n > 1));
         first += r.counts[i];
     }
     for (size_t i = 1; i < n; ++i) {
@@ -344,7 +346,7 @@ void engine_queue(dhx_engine* e, const dhx_launch* launches, size_t n, hipStream
     ensure_usable(e);
     for (size_t i = 0; i < n; ++i) validate(e, launches[i]);
     set_device(e);
-    for (size_t i = 0; i < n; ++i) hip_check(e, launch_one(e, launches[i], stream), "kernel launch");
+    for (size_t i = 0; i < n; ++i) hip_check(e, launch_one(e, launches[i], stream, false), "kernel launch");
 }
 
 void* engine_staging_in(dhx_engine* e, uint32_t slot) {
@@ -726,6 +728,7 @@ int dhx_launch_timings(dhx_engine* e, uint64_t batch, uint32_t iters, double* ms
         auto it = e->graphs.find(batch);
         if (it == e->graphs.end()) throw dhx::Error("batch has not been prepared");
         const auto& list = it->second.launches;
+        const bool shared = it->second.counts.size() > 1;
         if (count) *count = list.size();
         if (capacity < list.size()) throw dhx::Error("timing output too small");
         if (iters == 0) throw dhx::Error("iters must be positive");
@@ -734,9 +737,9 @@ int dhx_launch_timings(dhx_engine* e, uint64_t batch, uint32_t iters, double* ms
         hip_check(e, hipEventCreate(&a), "hipEventCreate");
         hip_check(e, hipEventCreate(&b), "hipEventCreate");
         for (size_t i = 0; i < list.size(); ++i) {
-            hip_check(e, launch_one(e, list[i], e->stream), "kernel launch");  // warm
+            hip_check(e, launch_one(e, list[i], e->stream, shared), "kernel launch");  // warm
             hip_check(e, hipEventRecord(a, e->stream), "hipEventRecord");
-            for (uint32_t k = 0; k < iters; ++k) hip_check(e, launch_one(e, list[i], e->stream), "kernel launch");
+            for (uint32_t k = 0; k < iters; ++k) hip_check(e, launch_one(e, list[i], e->stream, shared), "kernel launch");
             hip_check(e, hipEventRecord(b, e->stream), "hipEventRecord");
             hip_check(e, hipEventSynchronize(b), "hipEventSynchronize");
             float ms = 0.f;

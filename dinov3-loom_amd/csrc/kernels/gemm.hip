@@ -44,6 +44,12 @@ constexpr int kSwigluSplit4Rows = 8192;
 static_assert(SwigluTile::BK == SwigluTileS::BK, "one stage depth for every SwiGLU tile shape");
 using SplitTile = Tile<128, 128, 4, 1>;
 
+// Tiles of the ring kernels, two to eight waves of 32x32 or 32x64.
+using ResidRing32 = Tile<32, 64, 1, 2, 128>;
+using ResidRing64 = Tile<64, 64, 2, 2, 64>;
+using ResidRing128 = Tile<128, 64, 4, 2, 64>;
+constexpr int kRound = 256;  // workgroups of one per CU
+
 template <class T, class Args>
 hipError_t launch(void (*kernel)(Args), int tiles, const Args& a, hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3(gemm::tile_grid(tiles)), dim3(T::THREADS), 0, s, a);
@@ -73,7 +79,32 @@ hipError_t launch_qkv_rope(const QkvArgs& a, hipStream_t s) {
     return rows < kQkvSmallRows ? launch_qkv_tiles<QkvTileS>(a, s) : launch_qkv_tiles<QkvTile>(a, s);
 }
 
+template <class T, int NST, int K>
+static hipError_t launch_resid_ring(const ResidArgs& a, hipStream_t s) {
+    const int tiles = tiles_for<T>(a.rows, kHidden);
+    return a.stats ? launch<T>(gemm::resid_ring_kernel<T, NST, true, K / T::BK>, tiles, a, s)
+                   : launch<T>(gemm::resid_ring_kernel<T, NST, false, K / T::BK>, tiles, a, s);
+}
+
 hipError_t launch_resid(const ResidArgs& a, hipStream_t s) {
+    // Launches that one round of workgroups covers, one per CU, take the
+    // smallest ring tile that does (N = 384 is six 64-column tiles): a smaller
+    // one needs a second round, a larger one leaves CUs idle. Whole forward
+    // (one chain, graph replay): 32x64 for the o-projection at 201 rows 412 ->
+    // 403 us, 64x64 406; 64x64 for the down projection at 201 / 1005 / 2412
+    // rows 412 -> 376, 404 -> 368, 488 -> 455 us (32x64: 375, 367, 517), at
+    // 3216 rows 528 -> 551; 128x64 there 528 -> 517 and at 4020 rows 539 -> 527.
+    // Beside another image group's kernels (a.shared) the 128x64 ring, which
+    // takes a CU's LDS whole, loses to the tiles below (705 -> 742 us at 2 x
+    // 3216 rows).
+    const int round = a.rows <= kRound / 6 * 32   ? 32
+                      : a.rows <= kRound / 6 * 64 ? 64
+                      : a.rows <= kRound / 6 * 128 && !a.shared ? 128 : 0;
+    if (a.k == kHidden && round == 32) return launch_resid_ring<ResidRing32, 4, kHidden>(a, s);
+    if (a.k == kHidden && round == 64) return launch_resid_ring<ResidRing64, 5, kHidden>(a, s);
+    if (a.k == kHidden && round == 128) return launch_resid_ring<ResidRing128, 4, kHidden>(a, s);
+    if (a.k == kFF && (round == 32 || round == 64)) return launch_resid_ring<ResidRing64, 5, kFF>(a, s);
+    if (a.k == kFF && round == 128) return launch_resid_ring<ResidRing128, 4, kFF>(a, s);
     // The K loop walks its stages six at a time (gemm_main_dma).
     if (a.k % (6 * ResidTile::BK) != 0) return hipErrorInvalidValue;
     if (a.k == kHidden) {  // the o-projection: three 128-deep stages, unrolled

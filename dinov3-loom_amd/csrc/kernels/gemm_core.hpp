@@ -436,6 +436,131 @@ __device__ __forceinline__ void gemm_tile_dma(AL (&al)[2], WD& wd, half_t* b0, h
     epi(acc, m0, n0);
 }
 
+// Copies BYTES (rounded up to 1 KB) from the start of a buffer descriptor to
+// LDS with DMA loads, the 1 KB pieces spread over the waves (the last waves
+// repeat the last piece where they do not split evenly). Bytes past the
+// descriptor's end arrive as zeros; `lds` holds dma_copy_bytes(BYTES).
+constexpr int dma_copy_bytes(int bytes) { return (bytes + 1023) / 1024 * 1024; }
+template <int BYTES, int WAVES>
+__device__ __forceinline__ void dma_copy(const __amdgpu_buffer_rsrc_t& r, void* lds, int tid) {
+    constexpr int PIECES = dma_copy_bytes(BYTES) / 1024, PER = (PIECES + WAVES - 1) / WAVES;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int c = min(wave * PER + i, PIECES - 1);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)((char*)lds + c * 1024), 16,
+                                                 (tid & 63) * 16, c * 1024, 0, 0);
+    }
+}
+
+// A descriptor over `bytes` from base (both uniform).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dma_src(const void* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, kBufferRsrcWord3);
+}
+
+// Both operands through LDS: a ring of NST stages, each the tile's BK-deep
+// slice of A and W in fragment order (A blocks first, then W blocks, 1 KB
+// each), filled by DMA loads only. With the stage count known at compile
+// time and no register loads among them, every wait is an exact count of
+// DMA loads (see above), and NST - 1 stages are in flight from the start.
+template <class T, int NST>
+struct Ring {
+    static constexpr int KS = T::BK / 16;
+    static constexpr int AB = T::BM / 32 * KS, WB = T::BN / 32 * KS;  // 1 KB blocks per stage
+    static constexpr int HALFS = (AB + WB) * 512;
+    // Blocks per wave; where they do not split evenly the last waves repeat
+    // the last block (the same data to the same place), which keeps every
+    // wave's count of loads, and so the waits, the same.
+    static constexpr int PA = (AB + T::WAVES - 1) / T::WAVES, PW = (WB + T::WAVES - 1) / T::WAVES, PER_WAVE = PA + PW;
+    static_assert(NST >= 2 && (NST - 1) * PER_WAVE <= 63, "vmcnt range");
+    __amdgpu_buffer_rsrc_t ra, rw;
+    int ksteps, mb_last;  // K / 16; the last 32-row block of A, from the tile's first
+    // a: [rows][k] frag, w: [n][k] frag; the descriptors cover the tile's
+    // rows and columns.
+    __device__ __forceinline__ Ring(const half_t* a, const half_t* w, int rows, int k, int m0, int n0) {
+        ksteps = k / 16;
+        mb_last = (rows + 31) / 32 - 1 - m0 / 32;
+        ra = dma_src(a + (size_t)(m0 / 32) * ksteps * 512, min(T::BM / 32, mb_last + 1) * ksteps * 1024);
+        rw = dma_src(w + (size_t)(n0 / 32) * ksteps * 512, T::BN / 32 * ksteps * 1024);
+    }
+    __device__ __forceinline__ void load(half_t* stage, int kt, int tid) const {
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane16 = (tid & 63) * 16;
+#pragma unroll
+        for (int b = 0; b < PA; ++b) {
+            const int blk = AB % T::WAVES ? min(wave * PA + b, AB - 1) : wave * PA + b;
+            const int mb = min(blk / KS, mb_last), ks = blk % KS;  // blocks past the rows repeat the last
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(stage + blk * 512), 16,
+                                                     lane16, (mb * ksteps + kt * KS + ks) * 1024, 0, 0);
+        }
+#pragma unroll
+        for (int b = 0; b < PW; ++b) {
+            const int blk = WB % T::WAVES ? min(wave * PW + b, WB - 1) : wave * PW + b;
+            const int nb = blk / KS, ks = blk % KS;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void*)(stage + (AB + blk) * 512),
+                                                     16, lane16, (nb * ksteps + kt * KS + ks) * 1024, 0, 0);
+        }
+    }
+    // The stage's MFMAs: the fragments of k-slice kk + 1 are read while kk
+    // computes.
+    __device__ __forceinline__ static void mma(const half_t* stage, int tid, Acc<T>& acc) {
+        const int wave = tid >> 6, wm = wave % T::WGM, wn = wave / T::WGM;
+        const half_t* const a_s = stage + wm * T::FM * KS * 512 + (tid & 63) * 8;
+        const half_t* const w_s = stage + (AB + wn * T::FN * KS) * 512 + (tid & 63) * 8;
+        half8_t af[2][T::FM], wf[2][T::FN];
+        auto fetch = [&](int kk, int b) {
+#pragma unroll
+            for (int j = 0; j < T::FM; ++j) af[b][j] = *(const half8_t*)(a_s + (j * KS + kk) * 512);
+#pragma unroll
+            for (int i = 0; i < T::FN; ++i) wf[b][i] = *(const half8_t*)(w_s + (i * KS + kk) * 512);
+        };
+        fetch(0, 0);
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+            if (kk + 1 < KS) fetch(kk + 1, (kk + 1) & 1);
+#pragma unroll
+            for (int i = 0; i < T::FN; ++i)
+#pragma unroll
+                for (int j = 0; j < T::FM; ++j) acc.v[i][j] = mfma32x32x16(wf[kk & 1][i], af[kk & 1][j], acc.v[i][j]);
+        }
+    }
+};
+
+// The stages of a ring in LDS, as separate variables: the compiler tells
+// distinct variables apart, so a read of one stage does not wait for the DMA
+// in flight into the others. Declares `half_t* const bufs[NST]`.
+#define DHX_RING_BUFS(T, NST)                                                                                 \
+    constexpr int kRingHalfs = Ring<T, NST>::HALFS;                                                           \
+    __shared__ __attribute__((aligned(16))) half_t ring0[kRingHalfs], ring1[kRingHalfs],                      \
+        ring2[NST > 2 ? kRingHalfs : 8], ring3[NST > 3 ? kRingHalfs : 8], ring4[NST > 4 ? kRingHalfs : 8],    \
+        ring5[NST > 5 ? kRingHalfs : 8];                                                                      \
+    static_assert(NST <= 6, "six ring variables");                                                            \
+    half_t* const bufs[6] = {ring0, ring1, ring2, ring3, ring4, ring5}
+
+// The K loop over a Ring: step s waits until stage s has landed for every
+// wave (only the DMA of later stages may be outstanding), issues the DMA of
+// stage s + NST - 1 into the buffer stage s - 1 was read from (every wave
+// finished with it before this barrier) and computes stage s. mid(acc, s)
+// runs before step s's MFMAs; the caller's earlier DMA loads have landed for
+// every wave by then, and what mid(acc, 0) writes to LDS is visible to every
+// wave from step 1 on.
+template <class T, int NST, int KT, class Mid>
+__device__ __forceinline__ void gemm_main_ring(const Ring<T, NST>& ring, half_t* const (&bufs)[6], Acc<T>& acc, Mid&& mid) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < T::FN; ++i)
+#pragma unroll
+        for (int j = 0; j < T::FM; ++j) acc.v[i][j] = float16_t{};
+    static_for<(KT < NST - 1 ? KT : NST - 1)>([&](auto S) { ring.load(bufs[decltype(S)::value], decltype(S)::value, tid); });
+    static_for<KT>([&](auto S) {
+        constexpr int s = decltype(S)::value;
+        constexpr int ahead = KT - 1 - s < NST - 2 ? KT - 1 - s : NST - 2;  // later stages in flight
+        vm_barrier<ahead * Ring<T, NST>::PER_WAVE>();
+        if constexpr (s + NST - 1 < KT) ring.load(bufs[(s + NST - 1) % NST], s + NST - 1, tid);
+        mid(acc, S);
+        Ring<T, NST>::mma(bufs[s % NST], tid, acc);
+    });
+}
+
 // Workgroups for a launch: one per tile (a persistent walk over several
 // tiles per resident workgroup measured slower: the hardware balances the
 // last wave of tiles better), rounded up to a multiple of 8 for xcd_tile.

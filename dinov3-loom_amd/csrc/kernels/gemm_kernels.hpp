@@ -306,12 +306,88 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
     });
 }
 
+// Fragment i of row block j of the wave's part of x (a row block past the
+// rows repeats the last one).
+template <class T>
+__device__ __forceinline__ half8_t* resid_frag(const ResidArgs& p, const Frag<T>& f, int mblocks, int j, int i) {
+    const int mb = min(f.m_base / 32 + j, mblocks - 1);
+    return (half8_t*)(p.x + ((size_t)mb * (kHidden / 16) + f.n_base / 16 + i) * 512 + (threadIdx.x & 63) * 8);
+}
+
+// Epilogue of the residual GEMMs: x += ls * acc + ls * b (cst[0] = ls * b,
+// cst[1] = ls of the tile's columns), with STATS also the row statistics of
+// the updated x. Each 16-column half of an MFMA result becomes a fragment in
+// registers (frag_swap), and x is read (xold, loaded before the K loop: each
+// element belongs to one tile, so nothing else writes it meanwhile) and
+// written fragment by fragment, 1 KB contiguous per wave access. A statistics
+// slot is 64 columns: waves of 32 columns come in pairs, and the second
+// hands its rounded values to the first through LDS (hand: 2 KB per row
+// block; every load must have landed), which then sums all 64 in the same
+// order as a 64-column wave.
+template <class T, bool STATS>
+__device__ __forceinline__ void resid_epilogue(const ResidArgs& p, const Acc<T>& acc,
+                                               const half8_t (&xold)[T::FM][T::TN / 16], const float (&cst)[2][T::BN],
+                                               const Frag<T>& f, int n0, int mblocks, half8_t* hand) {
+    static_assert(T::TN == 64 || (T::TN == 32 && T::WGN == 2 && T::FM == 1), "one statistics slot per wave or pair");
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < T::FM; ++j) {
+        const int m = f.m_base + j * 32 + f.l32;
+        const bool valid = m < p.rows;
+        float v[32];
+        half8_t h[T::TN / 16];
+#pragma unroll
+        for (int i = 0; i < T::FN; ++i) {
+            float4_t u[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int nt = f.col(i, g) - n0;  // column in the tile
+                const float4_t bl = *(const float4_t*)&cst[0][nt], l = *(const float4_t*)&cst[1][nt];
+                u[g] = group4(acc.v[i][j], g) * l + bl;
+            }
+            frag_swap(u[0], u[1]);
+            frag_swap(u[2], u[3]);
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                const half8_t old = xold[j][2 * i + kk];
+                half8_t& n = h[2 * i + kk];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    n[e] = (half_t)((float)old[e] + u[2 * kk][e]);
+                    n[e + 4] = (half_t)((float)old[e + 4] + u[2 * kk + 1][e]);
+                }
+                if (valid) *resid_frag(p, f, mblocks, j, 2 * i + kk) = n;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[(2 * i + kk) * 8 + e] = (float)n[e];
+            }
+        }
+        if constexpr (STATS && T::TN == 32) {
+            half8_t* const pair = hand + (f.m_base % T::BM) / 32 * 128;
+            const bool first = f.n_base % 64 == 0;  // uniform per wave
+            lds_barrier();                          // every wave is done reading the LDS behind hand
+            if (!first) {
+                pair[lane] = h[0];
+                pair[64 + lane] = h[1];
+            }
+            lds_barrier();
+            if (first) {
+#pragma unroll
+                for (int kk = 0; kk < 2; ++kk) {
+                    const half8_t other = pair[kk * 64 + lane];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[16 + kk * 8 + e] = (float)other[e];
+                }
+            }
+            if (first) pair_stats(p.stats, m, f.n_base / 64, v, f.hi, valid);
+        } else if constexpr (STATS) {
+            pair_stats(p.stats, m, f.n_base / 64, v, f.hi, valid);
+        }
+    }
+}
+
 // Residual GEMM: x += ls * (A W^T + b), in place on the f16 residual stream
 // in fragment order (with STATS, also the LayerNorm row statistics of the
-// updated x). The epilogue turns each 16-column half of an MFMA result into a
-// fragment in registers (frag_swap) and reads and writes x fragment by
-// fragment (1 KB contiguous per wave access); LDS holds only the weight
-// stages and the column constants.
+// updated x); LDS holds only the weight stages and the column constants.
 template <class T, bool STATS, int KT = 0>
 __global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel(ResidArgs p) {
     static_assert(T::TN % 64 == 0 && T::TM == 32, "whole statistics slots, one 32-row block per wave");
@@ -320,26 +396,21 @@ __global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel
     __shared__ __attribute__((aligned(16))) half_t wb0[T::WF_HALFS], wb1[T::WF_HALFS], wb2[T::WF_HALFS];
     __shared__ __attribute__((aligned(16))) float cst[2][T::BN];  // bias * ls, ls of the tile's columns
     constexpr int NT = kHidden / T::BN;
-    const int tid = threadIdx.x, lane = tid & 63, mblocks = (p.rows + 31) / 32;
+    const int tid = threadIdx.x, mblocks = (p.rows + 31) / 32;
     ActFrags<T> al[2];
     init_frags(al, p.a, p.rows, p.k);
     WeightDma<T> wd(p.w, kHidden, p.k);
     // The epilogue's own operands are loaded ahead of the K loop: the old x
-    // fragments of the wave's 32 x TN block (each x element belongs to one
-    // tile, so nothing else writes them meanwhile) and the column constants
-    // (into LDS).
-    half8_t xold[XF];
+    // fragments of the wave's 32 x TN block and the column constants (into
+    // LDS).
+    half8_t xold[1][XF];
     float cb = 0.f, cl = 0.f;
-    auto x_frag = [&](int m0, int n0, int i) {
-        const Frag<T> f(m0, n0);
-        const int mb = min(f.m_base / 32, mblocks - 1);  // a wave past the rows re-reads the last block
-        return p.x + ((size_t)mb * (kHidden / 16) + f.n_base / 16 + i) * 512 + lane * 8;
-    };
     gemm_tile_dma<T, 1, KT>(
         al, wd, wb0, wb1, wb2, NT, NT * ((p.rows + T::BM - 1) / T::BM), p.k / T::BK,
         [&](int m0, int n0) {
+            const Frag<T> f(m0, n0);
 #pragma unroll
-            for (int i = 0; i < XF; ++i) xold[i] = *(const half8_t*)x_frag(m0, n0, i);
+            for (int i = 0; i < XF; ++i) xold[0][i] = *resid_frag(p, f, mblocks, 0, i);
             if (tid < T::BN) {
                 cb = p.bias[n0 + tid];
                 cl = p.ls[n0 + tid];
@@ -352,42 +423,51 @@ __global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel
             }
         },
         [&](const Acc<T>& acc, int m0, int n0) {
-        const Frag<T> f(m0, n0);
-        if (f.m_base / 32 >= mblocks) return;  // uniform per wave
-        const int m = f.m_base + f.l32;
-        const bool valid = m < p.rows;
+            const Frag<T> f(m0, n0);
+            if (f.m_base / 32 >= mblocks) return;  // uniform per wave
+            resid_epilogue<T, STATS>(p, acc, xold, cst, f, n0, mblocks, nullptr);
+        });
+}
+
+// The residual GEMMs on a ring, for launches that fit one round of workgroups
+// (see the launcher). There the time is the latency of a chain of stage
+// loads, and of a workgroup's loads through its CU's 64 bytes per clock:
+// small tiles spread the bytes over the chip and NST - 1 stages in flight
+// hide the latency that resid_kernel, with its activations one step ahead,
+// waits for in every step. Down projection at 201 rows 8.5 -> 5.8 us, at 1608
+// rows 8.7 -> 6.0 us; o-projection 4.3 -> 3.6 and 4.45 -> 3.9 us (HIP events,
+// alone). The column constants come through LDS by DMA as well, so that the
+// old x fragments, used only after every load has landed, are the only
+// register loads.
+template <class T, int NST, bool STATS, int KT>
+__global__ __launch_bounds__(T::THREADS, 1) void resid_ring_kernel(ResidArgs p) {
+    static_assert(T::BN <= T::THREADS, "one thread per column constant");
+    DHX_RING_BUFS(T, NST);
+    __shared__ __attribute__((aligned(16))) float raw_b[dma_copy_bytes(T::BN * 4) / 4], raw_l[dma_copy_bytes(T::BN * 4) / 4];
+    __shared__ __attribute__((aligned(16))) float cst[2][T::BN];  // bias * ls, ls of the tile's columns
+    constexpr int NT = kHidden / T::BN;
+    const int tid = threadIdx.x, mblocks = (p.rows + 31) / 32;
+    const int t = xcd_tile(NT * ((p.rows + T::BM - 1) / T::BM));
+    if (t < 0) return;  // uniform per workgroup
+    const int n0 = (t % NT) * T::BN, m0 = (t / NT) * T::BM;
+    const Frag<T> f(m0, n0);
+    half8_t xold[T::FM][T::TN / 16];
 #pragma unroll
-        for (int s2 = 0; s2 < T::TN / 64; ++s2) {
-            float v[32];
+    for (int j = 0; j < T::FM; ++j)
 #pragma unroll
-            for (int i2 = 0; i2 < 2; ++i2) {
-                const int i = 2 * s2 + i2;  // 32-column MFMA tile of the wave
-                float4_t u[4];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int nt = f.col(i, g) - n0;  // column in the tile
-                    const float4_t bl = *(const float4_t*)&cst[0][nt], l = *(const float4_t*)&cst[1][nt];
-                    u[g] = group4(acc.v[i][0], g) * l + bl;
-                }
-                frag_swap(u[0], u[1]);
-                frag_swap(u[2], u[3]);
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) {
-                    const half8_t old = xold[2 * i + kk];
-                    half8_t h;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        h[e] = (half_t)((float)old[e] + u[2 * kk][e]);
-                        h[e + 4] = (half_t)((float)old[e + 4] + u[2 * kk + 1][e]);
-                    }
-                    if (valid) *(half8_t*)x_frag(m0, n0, 2 * i + kk) = h;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[(i2 * 2 + kk) * 8 + e] = (float)h[e];
-                }
-            }
-            if constexpr (STATS) pair_stats(p.stats, m, f.n_base / 64 + s2, v, f.hi, valid);
+        for (int i = 0; i < T::TN / 16; ++i) xold[j][i] = *resid_frag(p, f, mblocks, j, i);
+    compiler_fence();
+    dma_copy<T::BN * 4, T::WAVES>(dma_src(p.bias + n0, T::BN * 4), raw_b, tid);
+    dma_copy<T::BN * 4, T::WAVES>(dma_src(p.ls + n0, T::BN * 4), raw_l, tid);
+    const Ring<T, NST> ring(p.a, p.w, p.rows, p.k, m0, n0);
+    Acc<T> acc;
+    gemm_main_ring<T, NST, KT>(ring, bufs, acc, [&](Acc<T>&, auto S) {
+        if (decltype(S)::value == 0 && tid < T::BN) {
+            cst[0][tid] = raw_b[tid] * raw_l[tid];
+            cst[1][tid] = raw_l[tid];
         }
     });
+    resid_epilogue<T, STATS>(p, acc, xold, cst, f, n0, mblocks, (half8_t*)ring0);
 }
 
 // SwiGLU dual GEMM. W rows are packed as blocks of 32 gate rows followed by

@@ -100,6 +100,9 @@ struct ResidArgs {
     int rows;
     int k;
     float* stats = nullptr;  // optional: row statistics of the updated x
+    // Other kernels run beside this launch (concurrent image groups); chooses
+    // the tile shape only, not the result.
+    bool shared = false;
 };
 
 // act[rows][1536] frag = silu(h.Wg^T + bg) * (h.Wu^T + bu), h frag; W and b are packed

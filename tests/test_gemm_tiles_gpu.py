@@ -1,0 +1,52 @@
+"""Every tile shape of the GEMM launchers gives a row the same bits: launches
+at the edges of each shape's range of rows (one row, a ragged last block, the
+last count of a shape and the first of the next) against the first rows of one
+larger launch on the same data, alone and beside another launch. The larger
+launches are the ones the per-kernel tests compare with the oracle."""
+import numpy as np
+import pytest
+
+import dinov3_hrx as d
+
+from test_kernels_gpu import K_RESID, K_RESID_S, allocf, eng, f16, readf, up, upf, _keys  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def run(e, kernel, scalars, bindings, beside=None):
+    """One launch, or with `beside` as one of two branches of a plan."""
+    key = next(_keys)
+    if beside is None:
+        e.record(key, [(kernel, scalars, bindings)])
+    else:
+        e.record_branches(key, [[(kernel, scalars, bindings)], [(kernel, scalars, beside)]])
+    e.replay(key)
+    e.synchronize()
+
+
+@pytest.mark.parametrize("kdim", [384, 1536])
+def test_resid_rows_do_not_depend_on_the_tile(eng, kdim):  # noqa: F811
+    rng = np.random.default_rng(kdim)
+    most = 6000
+    a, x0 = f16(rng.normal(size=(most, kdim))), f16(rng.normal(size=(most, 384)) * 2 + 0.5)
+    w = upf(eng, f16(rng.normal(size=(384, kdim)) * 0.03))
+    b = up(eng, (rng.normal(size=384) * 0.1).astype(np.float32))
+    ls = up(eng, rng.uniform(0.5, 1.5, size=384).astype(np.float32))
+
+    def launch(rows, beside=False):
+        ar = upf(eng, a[:rows])
+        x, st = upf(eng, x0[:rows]), eng.allocate(rows * 48)
+        other = [ar, w, b, ls, upf(eng, x0[:rows]), eng.allocate(rows * 48)] if beside else None
+        run(eng, K_RESID_S, [rows, kdim], [ar, w, b, ls, x, st], other)
+        plain = upf(eng, x0[:rows])
+        run(eng, K_RESID, [rows, kdim], [ar, w, b, ls, plain])
+        y = readf(eng, x, rows, 384)
+        assert np.array_equal(readf(eng, plain, rows, 384), y)
+        return y, eng.read(st, np.float32, (rows, 12))
+
+    want, want_stats = launch(most)
+    for rows in (1, 32, 33, 65, 1344, 1345, 2688, 2689, 5376, 5377):
+        for beside in (False, True):
+            got, stats = launch(rows, beside)
+            assert np.array_equal(got, want[:rows]), (rows, beside)
+            assert np.array_equal(stats, want_stats[:rows]), (rows, beside)
