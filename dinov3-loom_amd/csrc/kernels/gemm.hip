@@ -18,8 +18,8 @@ using PatchTile = Tile<64, 128, 2, 2>;
 // LDS, not registers): four workgroups per CU, so a batch of 64 (909 tiles)
 // runs as one round of workgroups.
 using QkvTile = Tile<128, 128, 4, 1, 32>;
-// QKV for launches of fewer rows (batch 32's and 512x512 batch 8's image
-// groups, small batches): 128x64 tiles (one head per wave), twice the
+// QKV for launches of fewer rows (512x512 batch 8's image groups): 128x64
+// tiles (one head per wave), twice the
 // workgroups. Same stage depth, and the LayerNorm fold is applied in the
 // epilogue, so a row's result is bitwise the same on either shape.
 using QkvTileS = Tile<128, 64, 4, 1, 32>;
@@ -48,6 +48,9 @@ using SplitTile = Tile<128, 128, 4, 1>;
 using ResidRing32 = Tile<32, 64, 1, 2, 128>;
 using ResidRing64 = Tile<64, 64, 2, 2, 64>;
 using ResidRing128 = Tile<128, 64, 4, 2, 64>;
+using QkvRing64 = Tile<64, 64, 2, 1, 64>;
+using QkvRing64W = Tile<64, 128, 2, 2, 64>;
+using QkvRing128 = Tile<128, 128, 4, 2, 64>;
 constexpr int kRound = 256;  // workgroups of one per CU
 
 template <class T, class Args>
@@ -74,8 +77,26 @@ static hipError_t launch_qkv_tiles(const QkvArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+template <class T, int NST>
+static hipError_t launch_qkv_ring(const QkvArgs& a, hipStream_t s) {
+    const dim3 grid(gemm::tile_grid(tiles_for<T>(a.images * (a.grid * a.grid + kPrefix), 3 * kHidden)));
+    const size_t lds = gemm::rope_lds_bytes(a.grid);
+    if (a.stats) hipLaunchKernelGGL((gemm::qkv_ring_kernel<T, NST, true>), grid, dim3(T::THREADS), lds, s, a);
+    else hipLaunchKernelGGL((gemm::qkv_ring_kernel<T, NST, false>), grid, dim3(T::THREADS), lds, s, a);
+    return hipGetLastError();
+}
+
+// As for the residual GEMMs: the smallest ring tile that one round of
+// workgroups covers. Whole forward (one chain, graph replay), the tiles
+// below / 64x64 / 64x128 / 128x128: 201 rows 418 / 390 / 395 / 405 us, 603
+// rows 426 / 401 / 406 / 420, 1005 rows 411 / 434 / 400 / 415, 1608 rows 446
+// / 461 / 427 / 440, 2412 rows 466 / 509 / 481 / 453, 3216 rows 503 / 586 /
+// 519 / 487, 4020 rows 513 / 645 / 583 / 559.
 hipError_t launch_qkv_rope(const QkvArgs& a, hipStream_t s) {
     const int rows = a.images * (a.grid * a.grid + kPrefix);
+    if (rows <= kRound / 18 * 64) return launch_qkv_ring<QkvRing64, 5>(a, s);
+    if (rows <= kRound / 9 * 64) return launch_qkv_ring<QkvRing64W, 4>(a, s);
+    if (rows <= kRound / 9 * 128) return launch_qkv_ring<QkvRing128, 3>(a, s);
     return rows < kQkvSmallRows ? launch_qkv_tiles<QkvTileS>(a, s) : launch_qkv_tiles<QkvTile>(a, s);
 }
 

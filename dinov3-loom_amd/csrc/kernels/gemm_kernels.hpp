@@ -153,23 +153,109 @@ __device__ __forceinline__ void init_frags(ActFrags<T> (&al)[2], const half_t* a
 __host__ __device__ constexpr int rope_table_rows(int grid) { return (grid + 15) / 16 * 16; }
 __host__ __device__ constexpr int rope_lds_bytes(int grid) { return 4 * rope_table_rows(grid) * 16 * 4; }
 
-// Wave w (0..3) fills table w (cos row part, sin row part, cos column part,
-// sin column part) with DMA loads of 16 table rows each: lane i moves 16
-// bytes, channels 4(i % 4) .. +3 of table row 16q + i / 4, to LDS byte
+// Table w (cos row part, sin row part, cos column part, sin column part) is
+// filled by wave w % WAVES with DMA loads of 16 table rows each: lane i moves
+// 16 bytes, channels 4(i % 4) .. +3 of table row 16q + i / 4, to LDS byte
 // 16i of the load's 1 KB. Rows past the grid read beyond the source table's
 // bounds, which the buffer descriptor turns into zeros, or other patches'
 // angles (grids under 16), and are never read back.
+template <int WAVES>
 __device__ __forceinline__ void rope_table_dma(const float* cos, const float* sin, int grid, float* lds, int tid) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int rows = rope_table_rows(grid);
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(wave & 1 ? sin : cos), 0, grid * grid * kHeadDim * 4, kBufferRsrcWord3);
-    float* const table = lds + wave * rows * 16;
-    for (int q = 0; q < rows / 16; ++q) {  // uniform, 1..4
-        const int row = q * 16 + (lane >> 2);
-        const int src = (wave < 2 ? row * grid * kHeadDim : row * kHeadDim + 16) + (lane & 3) * 4;  // floats
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(table + q * 256), 16,
-                                                 src * 4, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < (4 + WAVES - 1) / WAVES; ++i) {
+        const int w = wave + i * WAVES;  // uniform
+        if (w >= 4) break;
+        const __amdgpu_buffer_rsrc_t r = dma_src(w & 1 ? sin : cos, grid * grid * kHeadDim * 4);
+        float* const table = lds + w * rows * 16;
+        for (int q = 0; q < rows / 16; ++q) {  // uniform, 1..4
+            const int row = q * 16 + (lane >> 2);
+            const int src = (w < 2 ? row * grid * kHeadDim : row * kHeadDim + 16) + (lane & 3) * 4;  // floats
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(table + q * 256), 16,
+                                                     src * 4, 0, 0, 0);
+        }
+    }
+}
+
+// Epilogue of the QKV GEMM (see qkv_rope_kernel): bias and wsum hold the
+// tile's columns, rope_lds the tables of rope_table_dma, norm(j) is the
+// LayerNorm (mean, rstd) of this lane's row of row block j.
+template <class T, bool LN, class Norm>
+__device__ __forceinline__ void qkv_epilogue(const QkvArgs& p, const Acc<T>& acc, const Frag<T>& f, int m0, int n0,
+                                             const float* bias, const float* wsum, const float* rope_lds, Norm&& norm) {
+    const int P = p.grid * p.grid, Tok = P + kPrefix, M = p.images * Tok;
+    const int part = f.n_base / kHidden, head0 = (f.n_base % kHidden) / kHeadDim;
+    half_t* const out = part == 0 ? p.q : part == 1 ? p.k : p.v;
+    const size_t head_elems = (size_t)p.tpad * kHeadDim;
+    const int rows16 = rope_table_rows(p.grid);
+    // The tile's rows lie in images img0 .. img0 + BM / Tok + 1 (img0
+    // from the tile origin, so it is uniform); the descriptor covers
+    // those.
+    const int img0 = min(m0, M - 1) / Tok;
+    const int span = min(p.images - img0, T::BM / Tok + 2);
+    const WtOut wo(out + (size_t)img0 * kHeads * head_elems, (uint32_t)(span * kHeads * head_elems * 2));
+#pragma unroll
+    for (int j = 0; j < T::FM; ++j) {
+        const int mr = f.row(j);
+        const int m = min(mr, M - 1);  // rows past M are computed but never written out
+        const int img = m / Tok, tok = m - img * Tok;
+        // This row's angles (cos, sin of channels 8g + 4hi .. +3, g =
+        // 0..3); v tiles and prefix rows rotate by cos 1, sin 0.
+        const bool rot = part < 2 && tok >= kPrefix;
+        const int pt = max(tok - kPrefix, 0), gy = pt / p.grid, gx = pt - gy * p.grid;
+        float4_t co[4], si[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int at = (g < 2 ? gy * 16 : 2 * rows16 * 16 + gx * 16) + (g & 1) * 8 + f.hi * 4;
+            const float4_t c4 = *(const float4_t*)&rope_lds[at], s4 = *(const float4_t*)&rope_lds[at + rows16 * 16];
+            co[g] = rot ? c4 : float4_t{1.f, 1.f, 1.f, 1.f};
+            si[g] = rot ? s4 : float4_t{};
+        }
+        const RowNorm rn = norm(j);
+#pragma unroll
+        for (int h2 = 0; h2 < T::TN / kHeadDim; ++h2) {
+            half4_t lo_h[4], up_h[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int c = g * 8 + f.hi * 4;  // channel in the head (0..31); partner c + 32
+                const int nl = f.n_base - n0 + h2 * kHeadDim + c;  // column in the tile
+                float4_t lo = group4(acc.v[2 * h2][j], g), up = group4(acc.v[2 * h2 + 1][j], g);
+                const float4_t b_lo = *(const float4_t*)&bias[nl], b_up = *(const float4_t*)&bias[nl + 32];
+                float4_t w_lo{}, w_up{};
+                if constexpr (LN) {
+                    w_lo = *(const float4_t*)&wsum[nl];
+                    w_up = *(const float4_t*)&wsum[nl + 32];
+                }
+                // Explicit FMAs: a row's result is the same on every tile
+                // shape, however the compiler would contract each.
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (LN) {
+                        lo[e] = fmaf(fmaf(-rn.mean, w_lo[e], lo[e]), rn.rstd, b_lo[e]);
+                        up[e] = fmaf(fmaf(-rn.mean, w_up[e], up[e]), rn.rstd, b_up[e]);
+                    } else {
+                        lo[e] += b_lo[e];
+                        up[e] += b_up[e];
+                    }
+                    const float l = lo[e];
+                    lo[e] = fmaf(l, co[g][e], -(up[e] * si[g][e]));  // x[c] cos - x[c+32] sin
+                    up[e] = fmaf(up[e], co[g][e], l * si[g][e]);     // x[c+32] cos + x[c] sin
+                }
+                lo_h[g] = to_half4(lo);
+                up_h[g] = to_half4(up);
+            }
+            // Channels 16kk + 8hi .. +7 of the head for kk = 0..3.
+            const half8_t c0 = frag_swap(lo_h[0], lo_h[1]), c1 = frag_swap(lo_h[2], lo_h[3]);
+            const half8_t c2 = frag_swap(up_h[0], up_h[1]), c3 = frag_swap(up_h[2], up_h[3]);
+            const uint32_t hm = (uint32_t)(((img - img0) * kHeads + head0 + h2) * head_elems) * 2;
+            if (mr < M) {
+                wo.store(hm + (uint32_t)frag_piece(tok, f.hi * 8, kHeadDim) * 2, c0);
+                wo.store(hm + (uint32_t)frag_piece(tok, 16 + f.hi * 8, kHeadDim) * 2, c1);
+                wo.store(hm + (uint32_t)frag_piece(tok, 32 + f.hi * 8, kHeadDim) * 2, c2);
+                wo.store(hm + (uint32_t)frag_piece(tok, 48 + f.hi * 8, kHeadDim) * 2, c3);
+            }
+        }
     }
 }
 
@@ -189,8 +275,7 @@ template <class T, bool LN>
 __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2) void qkv_rope_kernel(QkvArgs p) {
     static_assert(T::TN % kHeadDim == 0 && kHidden % T::BN == 0 && T::WGN == 1,
                   "whole heads per wave and tile, whole rows per wave");
-    static_assert(T::WAVES == 4, "four waves fill the four RoPE tables");
-    __shared__ __attribute__((aligned(16))) half_t wb0[T::WF_HALFS], wb1[T::WF_HALFS], wb2[T::WF_HALFS];
+        __shared__ __attribute__((aligned(16))) half_t wb0[T::WF_HALFS], wb1[T::WF_HALFS], wb2[T::WF_HALFS];
     __shared__ __attribute__((aligned(16))) float cst[2][T::BN];  // bias, wsum of the tile's columns
     __shared__ float2_t rows_norm[T::BM];                          // (mean, rstd) of the tile's rows
     extern __shared__ __attribute__((aligned(16))) float rope_lds[];  // rope_table_dma's four tables
@@ -210,7 +295,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
     gemm_tile_dma<T, 1, kHidden / T::BK>(
         al, wd, wb0, wb1, wb2, NT, NT * ((M + T::BM - 1) / T::BM), kHidden / T::BK,
         [&](int m0, int n0) {
-            rope_table_dma(p.cos, p.sin, p.grid, rope_lds, tid);
+            rope_table_dma<T::WAVES>(p.cos, p.sin, p.grid, rope_lds, tid);
             const Frag<T> f(m0, n0);
             if constexpr (LN) {
 #pragma unroll
@@ -242,68 +327,52 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
         },
         [&](const Acc<T>& acc, int m0, int n0) {
         const Frag<T> f(m0, n0);
-        const int part = f.n_base / kHidden, head0 = (f.n_base % kHidden) / kHeadDim;
-        half_t* const out = part == 0 ? p.q : part == 1 ? p.k : p.v;
-        const size_t head_elems = (size_t)p.tpad * kHeadDim;
-        const int rows16 = rope_table_rows(p.grid);
-        // The tile's rows lie in images img0 .. img0 + BM / Tok + 1 (img0
-        // from the tile origin, so it is uniform); the descriptor covers
-        // those.
-        const int img0 = min(m0, M - 1) / Tok;
-        const int span = min(p.images - img0, T::BM / Tok + 2);
-        const WtOut wo(out + (size_t)img0 * kHeads * head_elems, (uint32_t)(span * kHeads * head_elems * 2));
+        qkv_epilogue<T, LN>(p, acc, f, m0, n0, cst[0], cst[1], rope_lds, [&](int j) {
+            if constexpr (!LN) return RowNorm{0.f, 1.f};
+            const float2_t v = rows_norm[f.m_base - m0 + j * 32 + f.l32];
+            return RowNorm{v[0], v[1]};
+        });
+    });
+}
+
+// The QKV GEMM on a ring, for launches that fit one round of workgroups (see
+// the launcher and resid_ring_kernel): everything the epilogue needs comes
+// through LDS by DMA ahead of the stages. In a forward the launch starts with
+// cold L2s, and qkv_rope_kernel's twelve 32-deep steps then each wait for a
+// load; here up to four 64-deep stages are in flight. At 201 rows 5.1 -> 4.7
+// us alone with warm caches, 2.3 us per launch less in the forward.
+template <class T, int NST, bool LN>
+__global__ __launch_bounds__(T::THREADS, 1) void qkv_ring_kernel(QkvArgs p) {
+    static_assert(T::TN % kHeadDim == 0 && kHidden % T::BN == 0, "whole heads per wave and tile");
+    DHX_RING_BUFS(T, NST);
+    __shared__ __attribute__((aligned(16))) float bias[dma_copy_bytes(T::BN * 4) / 4], wsum[dma_copy_bytes(T::BN * 4) / 4];
+    __shared__ __attribute__((aligned(16))) float stats[dma_copy_bytes(T::BM * kStatFloats * 4) / 4];
+    extern __shared__ __attribute__((aligned(16))) float rope_lds[];  // rope_table_dma's four tables
+    const int M = p.images * (p.grid * p.grid + kPrefix);
+    constexpr int NT = 3 * kHidden / T::BN;
+    const int tid = threadIdx.x;
+    const int t = xcd_tile(NT * ((M + T::BM - 1) / T::BM));
+    if (t < 0) return;  // uniform per workgroup
+    const int n0 = (t % NT) * T::BN, m0 = (t / NT) * T::BM;
+    const Frag<T> f(m0, n0);
+    rope_table_dma<T::WAVES>(p.cos, p.sin, p.grid, rope_lds, tid);
+    dma_copy<T::BN * 4, T::WAVES>(dma_src(p.bias + n0, T::BN * 4), bias, tid);
+    if constexpr (LN) {
+        dma_copy<T::BN * 4, T::WAVES>(dma_src(p.wsum + n0, T::BN * 4), wsum, tid);
+        dma_copy<T::BM * kStatFloats * 4, T::WAVES>(
+            dma_src(p.stats + (size_t)m0 * kStatFloats, min(T::BM, M - m0) * kStatFloats * 4), stats, tid);
+    }
+    const Ring<T, NST> ring(p.h, p.w, M, kHidden, m0, n0);
+    RowNorm rn[T::FM];
+    Acc<T> acc;
+    gemm_main_ring<T, NST, kHidden / T::BK>(ring, bufs, acc, [&](Acc<T>&, auto S) {
+        if constexpr (LN && decltype(S)::value == 0) {
 #pragma unroll
-        for (int j = 0; j < T::FM; ++j) {
-            const int mr = f.row(j);
-            const int m = min(mr, M - 1);  // rows past M are computed but never written out
-            const int img = m / Tok, tok = m - img * Tok;
-            // This row's angles (cos, sin of channels 8g + 4hi .. +3, g =
-            // 0..3); v tiles and prefix rows rotate by cos 1, sin 0.
-            const bool rot = part < 2 && tok >= kPrefix;
-            const int pt = max(tok - kPrefix, 0), gy = pt / p.grid, gx = pt - gy * p.grid;
-            float4_t co[4], si[4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int at = (g < 2 ? gy * 16 : 2 * rows16 * 16 + gx * 16) + (g & 1) * 8 + f.hi * 4;
-                const float4_t c4 = *(const float4_t*)&rope_lds[at], s4 = *(const float4_t*)&rope_lds[at + rows16 * 16];
-                co[g] = rot ? c4 : float4_t{1.f, 1.f, 1.f, 1.f};
-                si[g] = rot ? s4 : float4_t{};
-            }
-            RowNorm rn{0.f, 1.f};
-            if constexpr (LN) {
-                const float2_t v = rows_norm[f.m_base - m0 + j * 32 + f.l32];
-                rn = RowNorm{v[0], v[1]};
-            }
-#pragma unroll
-            for (int h2 = 0; h2 < T::TN / kHeadDim; ++h2) {
-                half4_t lo_h[4], up_h[4];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int c = g * 8 + f.hi * 4;  // channel in the head (0..31); partner c + 32
-                    const int nl = f.n_base - n0 + h2 * kHeadDim + c;  // column in the tile
-                    float4_t lo = group4(acc.v[2 * h2][j], g), up = group4(acc.v[2 * h2 + 1][j], g);
-                    if constexpr (LN) {
-                        lo = (lo - rn.mean * *(const float4_t*)&cst[1][nl]) * rn.rstd;
-                        up = (up - rn.mean * *(const float4_t*)&cst[1][nl + 32]) * rn.rstd;
-                    }
-                    lo += *(const float4_t*)&cst[0][nl];
-                    up += *(const float4_t*)&cst[0][nl + 32];
-                    lo_h[g] = to_half4(lo * co[g] - up * si[g]);  // x[c] cos - x[c+32] sin
-                    up_h[g] = to_half4(up * co[g] + lo * si[g]);  // x[c+32] cos + x[c] sin
-                }
-                // Channels 16kk + 8hi .. +7 of the head for kk = 0..3.
-                const half8_t c0 = frag_swap(lo_h[0], lo_h[1]), c1 = frag_swap(lo_h[2], lo_h[3]);
-                const half8_t c2 = frag_swap(up_h[0], up_h[1]), c3 = frag_swap(up_h[2], up_h[3]);
-                const uint32_t hm = (uint32_t)(((img - img0) * kHeads + head0 + h2) * head_elems) * 2;
-                if (mr < M) {
-                    wo.store(hm + (uint32_t)frag_piece(tok, f.hi * 8, kHeadDim) * 2, c0);
-                    wo.store(hm + (uint32_t)frag_piece(tok, 16 + f.hi * 8, kHeadDim) * 2, c1);
-                    wo.store(hm + (uint32_t)frag_piece(tok, 32 + f.hi * 8, kHeadDim) * 2, c2);
-                    wo.store(hm + (uint32_t)frag_piece(tok, 48 + f.hi * 8, kHeadDim) * 2, c3);
-                }
-            }
+            for (int j = 0; j < T::FM; ++j) rn[j] = row_norm(stats, f.row(j) - m0);
         }
     });
+    qkv_epilogue<T, LN>(p, acc, f, m0, n0, bias, wsum, rope_lds,
+                        [&](int j) { return LN ? rn[j] : RowNorm{0.f, 1.f}; });
 }
 
 // Fragment i of row block j of the wave's part of x (a row block past the

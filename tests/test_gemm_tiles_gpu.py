@@ -6,9 +6,10 @@ launches are the ones the per-kernel tests compare with the oracle."""
 import numpy as np
 import pytest
 
-import dinov3_hrx as d
+import oracle
 
-from test_kernels_gpu import K_RESID, K_RESID_S, allocf, eng, f16, readf, up, upf, _keys  # noqa: F401
+from test_kernels_gpu import (K_QKV, K_QKV_LN, K_RESID, K_RESID_S, allocf, eng, f16, read_heads, readf,  # noqa: F401
+                              slot_stats, up, upf, _keys)
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,29 @@ def test_resid_rows_do_not_depend_on_the_tile(eng, kdim):  # noqa: F811
             got, stats = launch(rows, beside)
             assert np.array_equal(got, want[:rows]), (rows, beside)
             assert np.array_equal(stats, want_stats[:rows]), (rows, beside)
+
+
+@pytest.mark.parametrize("grid,most,counts", [(4, 300, (1, 2, 42, 43, 85, 86, 170, 171)), (14, 26, (1, 4, 5, 8, 9, 17, 18)),
+                                              (59, 2, (1,))])
+def test_qkv_rows_do_not_depend_on_the_tile(eng, grid, most, counts):  # noqa: F811
+    rng = np.random.default_rng(grid)
+    T = grid * grid + 5
+    tpad = (T + 127) // 128 * 128
+    x = f16(rng.normal(size=(most * T, 384)) * 1.5 + 0.5)
+    w = upf(eng, f16(rng.normal(size=(1152, 384)) * 0.05))
+    wsum, b = (up(eng, (rng.normal(size=1152) * 0.1).astype(np.float32)) for _ in range(2))
+    cos, sin = (up(eng, t) for t in oracle.rope_tables(grid))
+
+    def launch(images):
+        xr, st, nb = upf(eng, x[:images * T]), up(eng, slot_stats(x[:images * T])), images * 6 * tpad * 64 * 2
+        got = []
+        for kernel, first in ((K_QKV, [xr, w, b]), (K_QKV_LN, [xr, st, w, wsum, b])):
+            out = [eng.allocate(nb) for _ in range(3)]
+            run(eng, kernel, [images, grid, tpad], first + [cos, sin] + out)
+            got += [read_heads(eng, r, images, tpad) for r in out]
+        return got
+
+    want = launch(most)
+    for images in counts:
+        for name, g, r in zip(("q", "k", "v", "q LN", "k LN", "v LN"), launch(images), want):
+            assert np.array_equal(g, r[:images]), (images, name)
