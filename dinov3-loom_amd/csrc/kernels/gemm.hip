@@ -48,6 +48,9 @@ using SplitTile = Tile<128, 128, 4, 1>;
 using ResidRing32 = Tile<32, 64, 1, 2, 128>;
 using ResidRing64 = Tile<64, 64, 2, 2, 64>;
 using ResidRing128 = Tile<128, 64, 4, 2, 64>;
+using SwigluRing64 = Tile<64, 128, 2, 2, 32>;
+using SwigluRing128 = Tile<128, 128, 4, 2, 32>;
+using SwigluRing128W = Tile<128, 192, 4, 3, 32>;
 using QkvRing64 = Tile<64, 64, 2, 1, 64>;
 using QkvRing64W = Tile<64, 128, 2, 2, 64>;
 using QkvRing128 = Tile<128, 128, 4, 2, 64>;
@@ -157,11 +160,31 @@ static hipError_t launch_swiglu_tiles(const SwigluArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// The XCD split (each XCD's L2 keeps 1/NS of the weights): two N slices for
+template <class T, int NST>
+static hipError_t launch_swiglu_ring(const SwigluArgs& a, hipStream_t s) {
+    const dim3 grid(gemm::tile_grid(tiles_for<T>(a.rows, 2 * kFF)));
+    if (a.stats) hipLaunchKernelGGL((gemm::swiglu_ring_kernel<T, NST, true>), grid, dim3(T::THREADS), 0, s, a);
+    else hipLaunchKernelGGL((gemm::swiglu_ring_kernel<T, NST, false>), grid, dim3(T::THREADS), 0, s, a);
+    return hipGetLastError();
+}
+
+// As for the residual GEMMs: the smallest ring tile that one round of
+// workgroups covers, to 2048 rows. Whole forward (one chain, graph replay),
+// the 128x128 tiles below / 64x128 / 128x128 / 128x192 rings: 201 rows 336 /
+// 329 / 336 / - us, 603 rows 345 / 337 / 343 / -, 1005 rows 349 / 355 / 346 /
+// -, 1206 rows 375 / 359 / 353 / -, 1608 rows 379 / - / 381 / 371, 2010 rows
+// 391 / - / 394 / 385, 2412 rows 404 / - / 407 / 457. Above, several rounds
+// overlap one tile's epilogue with another's K loop, which the rings, taking
+// most of a CU's LDS, do not.
+//
+// For the larger launches, the XCD split (each XCD's L2 keeps 1/NS of the weights): two N slices for
 // the whole batch-64 launch, four for the image groups of 5120 - 8191 rows
 // that the forward runs concurrently (measured: forward +0.9 % at batch 64,
 // the whole-batch launch 2 % slower with four).
 hipError_t launch_swiglu(const SwigluArgs& a, hipStream_t s) {
+    if (a.rows <= kRound / 24 * 64) return launch_swiglu_ring<SwigluRing64, 4>(a, s);
+    if (a.rows <= kRound / 24 * 128) return launch_swiglu_ring<SwigluRing128, 4>(a, s);
+    if (a.rows <= kRound / 16 * 128) return launch_swiglu_ring<SwigluRing128W, 4>(a, s);
     if (a.rows < kSwigluSmallRows) return launch_swiglu_tiles<SwigluTileS, 2>(a, s);
     return a.rows < kSwigluSplit4Rows ? launch_swiglu_tiles<SwigluTile, 4>(a, s) : launch_swiglu_tiles<SwigluTile, 2>(a, s);
 }

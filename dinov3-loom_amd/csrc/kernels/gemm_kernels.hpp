@@ -539,6 +539,65 @@ __global__ __launch_bounds__(T::THREADS, 1) void resid_ring_kernel(ResidArgs p) 
     resid_epilogue<T, STATS>(p, acc, xold, cst, f, n0, mblocks, (half8_t*)ring0);
 }
 
+// Epilogue of the SwiGLU GEMM (see swiglu_kernel): bias holds the tile's
+// column constants, gate columns scaled by -log2(e) and up columns by -ln(2).
+template <class T>
+__device__ __forceinline__ void swiglu_epilogue(const SwigluArgs& p, const Acc<T>& acc, const Frag<T>& f, int n0,
+                                                const float* bias, const RowNorm (&rn)[T::FM]) {
+    const int lane = threadIdx.x & 63, mblocks = (p.rows + 31) / 32;
+    // Pair q of the wave: gate = acc.v[2q], up = acc.v[2q + 1], outputs
+    // 32q .. 32q+31 of the wave's OW, i.e. act fragments 2q and 2q + 1.
+    // With gate g and up u (after LayerNorm folding and bias), the output
+    // silu(g) u = g u / (1 + e^-g) is computed from gs = -g log2(e) and
+    // us = -u ln(2) as gs us / (1 + 2^gs) (gs us = g u): the scales ride
+    // on the FMAs that apply rstd and the bias, which saves the multiply
+    // that would otherwise form the exponent.
+#pragma unroll
+    for (int j = 0; j < T::FM; ++j) {
+        const int mb = f.m_base / 32 + j;
+        if (mb >= mblocks) break;  // uniform per wave
+        const float sg = rn[j].rstd * -kLog2e, su = rn[j].rstd * -kLn2;
+        const WtOut act(p.act + (size_t)mb * (kFF / 16) * 512, 32 * kFF * 2);
+#pragma unroll
+        for (int q = 0; q < T::FN / 2; ++q) {
+            half4_t y[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int c = g * 8 + f.hi * 4, nl = f.n_base - n0 + 64 * q + c;
+                float4_t gate = group4(acc.v[2 * q][j], g), up = group4(acc.v[2 * q + 1][j], g);
+                const float4_t gs = gate * sg + *(const float4_t*)&bias[nl];
+                const float4_t us = up * su + *(const float4_t*)&bias[nl + 32];
+                float4_t r;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r[e] = gs[e] * us[e] * fast_rcp(1.0f + fast_exp2(gs[e]));
+                y[g] = to_half4(r);
+            }
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+                act.store(((f.n_base / 32 + 2 * q + kk) * 512 + lane * 8) * 2, frag_swap(y[2 * kk], y[2 * kk + 1]));
+        }
+    }
+}
+
+// The scale a column's bias is kept with (the first 32 of each 64 are gates).
+__device__ __forceinline__ float swiglu_scale(int column) { return column % 64 < 32 ? -kLog2e : -kLn2; }
+
+// Adds the folded LayerNorm's -mean * wsum to column block i of the
+// accumulators; wsum: the 32 columns of the block.
+template <class T>
+__device__ __forceinline__ void swiglu_mean(Acc<T>& acc, int i, const float* wsum, const RowNorm (&rn)[T::FM]) {
+    const int hi = (threadIdx.x & 63) >> 5;
+    float4_t w[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) w[g] = *(const float4_t*)&wsum[8 * g + 4 * hi];
+#pragma unroll
+    for (int j = 0; j < T::FM; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc.v[i][j][4 * g + e] = fmaf(-rn[j].mean, w[g][e], acc.v[i][j][4 * g + e]);
+}
+
 // SwiGLU dual GEMM. W rows are packed as blocks of 32 gate rows followed by
 // the 32 matching up rows, so a wave's 128 columns are two gate/up pairs of
 // 32 outputs each. The tile's column constants (bias, and wsum with the
@@ -583,9 +642,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(
         },
         [&] {
             if (tid < T::BN) {
-                // Gate columns (the first 32 of each 64) are kept scaled by
-                // -log2(e), up columns by -ln(2); see the epilogue.
-                cst[0][tid] = cb * (tid % 64 < 32 ? -kLog2e : -kLn2);
+                cst[0][tid] = cb * swiglu_scale(tid);
                 cst[1][tid] = cw;
             }
 #pragma unroll
@@ -593,39 +650,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(
         },
         [&](const Acc<T>& acc, int m0, int n0) {
         const Frag<T> f(m0, n0);
-        const int lane = threadIdx.x & 63, mblocks = (p.rows + 31) / 32;
-        // Pair q of the wave: gate = acc.v[2q], up = acc.v[2q + 1], outputs
-        // 32q .. 32q+31 of the wave's OW, i.e. act fragments 2q and 2q + 1.
-        // With gate g and up u (after LayerNorm folding and bias), the output
-        // silu(g) u = g u / (1 + e^-g) is computed from gs = -g log2(e) and
-        // us = -u ln(2) as gs us / (1 + 2^gs) (gs us = g u): the scales ride
-        // on the FMAs that apply rstd and the bias, which saves the multiply
-        // that would otherwise form the exponent.
-#pragma unroll
-        for (int j = 0; j < T::FM; ++j) {
-            const int mb = f.m_base / 32 + j;
-            if (mb >= mblocks) break;  // uniform per wave
-            const float sg = rn[j].rstd * -kLog2e, su = rn[j].rstd * -kLn2;
-            const WtOut act(p.act + (size_t)mb * (kFF / 16) * 512, 32 * kFF * 2);
-#pragma unroll
-            for (int q = 0; q < T::FN / 2; ++q) {
-                half4_t y[4];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int c = g * 8 + f.hi * 4, nl = f.n_base - n0 + 64 * q + c;
-                    float4_t gate = group4(acc.v[2 * q][j], g), up = group4(acc.v[2 * q + 1][j], g);
-                    const float4_t gs = gate * sg + *(const float4_t*)&cst[0][nl];
-                    const float4_t us = up * su + *(const float4_t*)&cst[0][nl + 32];
-                    float4_t r;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) r[e] = gs[e] * us[e] * fast_rcp(1.0f + fast_exp2(gs[e]));
-                    y[g] = to_half4(r);
-                }
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk)
-                    act.store(((f.n_base / 32 + 2 * q + kk) * 512 + lane * 8) * 2, frag_swap(y[2 * kk], y[2 * kk + 1]));
-            }
-        }
+        swiglu_epilogue<T>(p, acc, f, n0, cst[0], rn);
     },
     // The folded LayerNorm's -mean * wsum, added to column block i of the
     // accumulators at step i + 1 of the K loop (an additive term may join
@@ -635,22 +660,56 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(
         if constexpr (LN) {
             static_for<T::FN>([&](auto I) {
                 constexpr int i = decltype(I)::value;
-                if (s == i + 1) {
-                    const int hi = (threadIdx.x & 63) >> 5;
-                    float4_t w[4];
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) w[g] = *(const float4_t*)&cst[1][32 * i + 8 * g + 4 * hi];
-#pragma unroll
-                    for (int j = 0; j < T::FM; ++j)
-#pragma unroll
-                        for (int g = 0; g < 4; ++g)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                acc.v[i][j][4 * g + e] = fmaf(-rn[j].mean, w[g][e], acc.v[i][j][4 * g + e]);
-                }
+                if (s == i + 1) swiglu_mean<T>(acc, i, &cst[1][32 * i], rn);
             });
         }
     });
+}
+
+// The SwiGLU GEMM on a ring, for launches that fit one round of workgroups
+// (see the launcher and resid_ring_kernel), its column constants and row
+// statistics through LDS by DMA; alone at 201 rows 5.3 -> 4.9 us, at 1206
+// rows 7.4 -> 5.7, at 1608 rows 7.4 -> 6.8. The folded LayerNorm's mean term joins column
+// block b (of each 128 columns) before K step 64(b + 1), as in swiglu_kernel,
+// so a row's result is bitwise the same on either.
+template <class T, int NST, bool LN>
+__global__ __launch_bounds__(T::THREADS, 1) void swiglu_ring_kernel(SwigluArgs p) {
+    static_assert(T::TN % 64 == 0, "whole gate/up pairs");
+    static_assert(T::BN <= T::THREADS && T::BK <= 64, "one thread per column constant");
+    DHX_RING_BUFS(T, NST);
+    __shared__ __attribute__((aligned(16))) float raw[dma_copy_bytes(T::BN * 4) / 4], wsum[dma_copy_bytes(T::BN * 4) / 4];
+    __shared__ __attribute__((aligned(16))) float stats[dma_copy_bytes(T::BM * kStatFloats * 4) / 4], bias[T::BN];
+    constexpr int NT = 2 * kFF / T::BN;
+    const int tid = threadIdx.x;
+    const int t = xcd_tile(NT * ((p.rows + T::BM - 1) / T::BM));
+    if (t < 0) return;  // uniform per workgroup
+    const int n0 = (t % NT) * T::BN, m0 = (t / NT) * T::BM;
+    const Frag<T> f(m0, n0);
+    dma_copy<T::BN * 4, T::WAVES>(dma_src(p.bias + n0, T::BN * 4), raw, tid);
+    if constexpr (LN) {
+        dma_copy<T::BN * 4, T::WAVES>(dma_src(p.wsum + n0, T::BN * 4), wsum, tid);
+        dma_copy<T::BM * kStatFloats * 4, T::WAVES>(
+            dma_src(p.stats + (size_t)m0 * kStatFloats, min(T::BM, p.rows - m0) * kStatFloats * 4), stats, tid);
+    }
+    const Ring<T, NST> ring(p.h, p.w, p.rows, kHidden, m0, n0);
+    const int nb = __builtin_amdgcn_readfirstlane(f.n_base / 32);  // first column block of the wave
+    RowNorm rn[T::FM];
+    Acc<T> acc;
+    gemm_main_ring<T, NST, kHidden / T::BK>(ring, bufs, acc, [&](Acc<T>& a, auto S) {
+        constexpr int s = decltype(S)::value;
+        if constexpr (s == 0) {
+            if (tid < T::BN) bias[tid] = raw[tid] * swiglu_scale(tid);
+#pragma unroll
+            for (int j = 0; j < T::FM; ++j) rn[j] = LN ? row_norm(stats, f.row(j) - m0) : RowNorm{0.f, 1.f};
+        }
+        if constexpr (LN && s > 0 && s * T::BK % 64 == 0 && s * T::BK <= 256) {
+            static_for<T::FN>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+                if ((nb + i) % 4 == s * T::BK / 64 - 1) swiglu_mean<T>(a, i, &wsum[f.n_base - n0 + 32 * i], rn);
+            });
+        }
+    });
+    swiglu_epilogue<T>(p, acc, f, n0, bias, rn);
 }
 
 // Split-K GEMM into f32 slabs [split][rows][384]; no atomics, so results do

@@ -8,8 +8,8 @@ import pytest
 
 import oracle
 
-from test_kernels_gpu import (K_QKV, K_QKV_LN, K_RESID, K_RESID_S, allocf, eng, f16, read_heads, readf,  # noqa: F401
-                              slot_stats, up, upf, _keys)
+from test_kernels_gpu import (K_QKV, K_QKV_LN, K_RESID, K_RESID_S, K_SWIGLU, K_SWIGLU_LN, _keys, allocf, eng,  # noqa: F401
+                              f16, read_heads, readf, slot_stats, up, upf)
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +77,24 @@ def test_qkv_rows_do_not_depend_on_the_tile(eng, grid, most, counts):  # noqa: F
     for images in counts:
         for name, g, r in zip(("q", "k", "v", "q LN", "k LN", "v LN"), launch(images), want):
             assert np.array_equal(g, r[:images]), (images, name)
+
+
+def test_swiglu_rows_do_not_depend_on_the_tile(eng):  # noqa: F811
+    rng = np.random.default_rng(8)
+    most = 8400
+    x = f16(rng.normal(size=(most, 384)) * 1.5 + 0.5)
+    w = upf(eng, f16(rng.normal(size=(3072, 384)) * 0.05))
+    wsum, b = (up(eng, (rng.normal(size=3072) * 0.1).astype(np.float32)) for _ in range(2))
+
+    def launch(rows):
+        xr, st, got = upf(eng, x[:rows]), up(eng, slot_stats(x[:rows])), []
+        for kernel, binds in ((K_SWIGLU, [xr, w, b]), (K_SWIGLU_LN, [xr, st, w, wsum, b])):
+            act = allocf(eng, rows, 1536)
+            run(eng, kernel, [rows], binds + [act])
+            got.append(readf(eng, act, rows, 1536))
+        return got
+
+    want = launch(most)
+    for rows in (1, 33, 640, 641, 1280, 1281, 2048, 2049, 5119, 5120):
+        for name, g, r in zip(("plain", "LN"), launch(rows), want):
+            assert np.array_equal(g, r[:rows]), (rows, name)
