@@ -207,10 +207,16 @@ __device__ __forceinline__ void qkv_epilogue(const QkvArgs& p, const Acc<T>& acc
         float4_t co[4], si[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int at = (g < 2 ? gy * 16 : 2 * rows16 * 16 + gx * 16) + (g & 1) * 8 + f.hi * 4;
-            const float4_t c4 = *(const float4_t*)&rope_lds[at], s4 = *(const float4_t*)&rope_lds[at + rows16 * 16];
-            co[g] = rot ? c4 : float4_t{1.f, 1.f, 1.f, 1.f};
-            si[g] = rot ? s4 : float4_t{};
+            co[g] = float4_t{1.f, 1.f, 1.f, 1.f};
+            si[g] = float4_t{};
+        }
+        if (rot) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int at = (g < 2 ? gy * 16 : 2 * rows16 * 16 + gx * 16) + (g & 1) * 8 + f.hi * 4;
+                co[g] = *(const float4_t*)&rope_lds[at];
+                si[g] = *(const float4_t*)&rope_lds[at + rows16 * 16];
+            }
         }
         const RowNorm rn = norm(j);
 #pragma unroll
@@ -375,12 +381,13 @@ __global__ __launch_bounds__(T::THREADS, 1) void qkv_ring_kernel(QkvArgs p) {
                         [&](int j) { return LN ? rn[j] : RowNorm{0.f, 1.f}; });
 }
 
-// Fragment i of row block j of the wave's part of x (a row block past the
-// rows repeats the last one).
+// This lane's piece of the first fragment of row block j of the wave's part
+// of x (a row block past the rows repeats the last one); the next fragments
+// follow 64 pieces apart.
 template <class T>
-__device__ __forceinline__ half8_t* resid_frag(const ResidArgs& p, const Frag<T>& f, int mblocks, int j, int i) {
+__device__ __forceinline__ half8_t* resid_frag(const ResidArgs& p, const Frag<T>& f, int mblocks, int j) {
     const int mb = min(f.m_base / 32 + j, mblocks - 1);
-    return (half8_t*)(p.x + ((size_t)mb * (kHidden / 16) + f.n_base / 16 + i) * 512 + (threadIdx.x & 63) * 8);
+    return (half8_t*)(p.x + ((size_t)mb * (kHidden / 16) + f.n_base / 16) * 512) + (threadIdx.x & 63);
 }
 
 // Epilogue of the residual GEMMs: x += ls * acc + ls * b (cst[0] = ls * b,
@@ -405,6 +412,7 @@ __device__ __forceinline__ void resid_epilogue(const ResidArgs& p, const Acc<T>&
         const bool valid = m < p.rows;
         float v[32];
         half8_t h[T::TN / 16];
+        half8_t* const x = resid_frag(p, f, mblocks, j);
 #pragma unroll
         for (int i = 0; i < T::FN; ++i) {
             float4_t u[4];
@@ -425,7 +433,7 @@ __device__ __forceinline__ void resid_epilogue(const ResidArgs& p, const Acc<T>&
                     n[e] = (half_t)((float)old[e] + u[2 * kk][e]);
                     n[e + 4] = (half_t)((float)old[e + 4] + u[2 * kk + 1][e]);
                 }
-                if (valid) *resid_frag(p, f, mblocks, j, 2 * i + kk) = n;
+                if (valid) x[(2 * i + kk) * 64] = n;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[(2 * i + kk) * 8 + e] = (float)n[e];
             }
@@ -479,7 +487,7 @@ __global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel
         [&](int m0, int n0) {
             const Frag<T> f(m0, n0);
 #pragma unroll
-            for (int i = 0; i < XF; ++i) xold[0][i] = *resid_frag(p, f, mblocks, 0, i);
+            for (int i = 0; i < XF; ++i) xold[0][i] = resid_frag(p, f, mblocks, 0)[i * 64];
             if (tid < T::BN) {
                 cb = p.bias[n0 + tid];
                 cl = p.ls[n0 + tid];
@@ -524,7 +532,7 @@ __global__ __launch_bounds__(T::THREADS, 1) void resid_ring_kernel(ResidArgs p) 
 #pragma unroll
     for (int j = 0; j < T::FM; ++j)
 #pragma unroll
-        for (int i = 0; i < T::TN / 16; ++i) xold[j][i] = *resid_frag(p, f, mblocks, j, i);
+        for (int i = 0; i < T::TN / 16; ++i) xold[j][i] = resid_frag(p, f, mblocks, j)[i * 64];
     compiler_fence();
     dma_copy<T::BN * 4, T::WAVES>(dma_src(p.bias + n0, T::BN * 4), raw_b, tid);
     dma_copy<T::BN * 4, T::WAVES>(dma_src(p.ls + n0, T::BN * 4), raw_l, tid);
