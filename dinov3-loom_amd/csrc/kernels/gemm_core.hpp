@@ -473,6 +473,11 @@ struct Ring {
     // wave's count of loads, and so the waits, the same.
     static constexpr int PA = (AB + T::WAVES - 1) / T::WAVES, PW = (WB + T::WAVES - 1) / T::WAVES, PER_WAVE = PA + PW;
     static_assert(NST >= 2 && (NST - 1) * PER_WAVE <= 63, "vmcnt range");
+    // Waves per SIMD that the stages (and about 6 KB beside them) leave room
+    // for, as the launch bound: with two, the accumulators stay in the
+    // architectural registers; bounded by one, the compiler keeps them in the
+    // others and copies them back and forth in the epilogue.
+    static constexpr int MIN_WAVES = 160 * 1024 / (NST * HALFS * 2 + 6 * 1024) * T::WAVES / 4 >= 2 ? 2 : 1;
     __amdgpu_buffer_rsrc_t ra, rw;
     int ksteps, mb_last;  // K / 16; the last 32-row block of A, from the tile's first
     // a: [rows][k] frag, w: [n][k] frag; the descriptors cover the tile's

@@ -348,7 +348,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
 // load; here up to four 64-deep stages are in flight. At 201 rows 5.1 -> 4.7
 // us alone with warm caches, 2.3 us per launch less in the forward.
 template <class T, int NST, bool LN>
-__global__ __launch_bounds__(T::THREADS, 1) void qkv_ring_kernel(QkvArgs p) {
+__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void qkv_ring_kernel(QkvArgs p) {
     static_assert(T::TN % kHeadDim == 0 && kHidden % T::BN == 0, "whole heads per wave and tile");
     DHX_RING_BUFS(T, NST);
     __shared__ __attribute__((aligned(16))) float bias[dma_copy_bytes(T::BN * 4) / 4], wsum[dma_copy_bytes(T::BN * 4) / 4];
@@ -517,7 +517,7 @@ __global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel
 // old x fragments, used only after every load has landed, are the only
 // register loads.
 template <class T, int NST, bool STATS, int KT>
-__global__ __launch_bounds__(T::THREADS, 1) void resid_ring_kernel(ResidArgs p) {
+__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void resid_ring_kernel(ResidArgs p) {
     static_assert(T::BN <= T::THREADS, "one thread per column constant");
     DHX_RING_BUFS(T, NST);
     __shared__ __attribute__((aligned(16))) float raw_b[dma_copy_bytes(T::BN * 4) / 4], raw_l[dma_copy_bytes(T::BN * 4) / 4];
@@ -681,7 +681,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(
 // block b (of each 128 columns) before K step 64(b + 1), as in swiglu_kernel,
 // so a row's result is bitwise the same on either.
 template <class T, int NST, bool LN>
-__global__ __launch_bounds__(T::THREADS, 1) void swiglu_ring_kernel(SwigluArgs p) {
+__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void swiglu_ring_kernel(SwigluArgs p) {
     static_assert(T::TN % 64 == 0, "whole gate/up pairs");
     static_assert(T::BN <= T::THREADS && T::BK <= 64, "one thread per column constant");
     DHX_RING_BUFS(T, NST);
