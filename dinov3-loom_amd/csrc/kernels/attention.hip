@@ -1,14 +1,17 @@
 // Online-softmax attention for gfx950 (replaces the reference's
 // kernels/attention_online_f16_wmma_cf16.loom).
 //
-// One workgroup = 4 waves = 128 queries of one (image, head); each wave owns
-// 32 queries. Keys stream through LDS in blocks of 32 or 64 (K and V both as
-// [key][ch]), so the same kernel serves 201 tokens (224x224) and 1029
-// tokens (512x512). q, k and v come per (image, head) as [tpad][64]
+// Three kernels share one step (attend32), each wave owning 32 queries of one
+// (image, head) and taking 32 keys a step: attention_kernel (four waves walk
+// all keys), attention_resident_kernel (the same with every key block in
+// flight at once, for short sequences in small launches) and
+// attention_split_kernel (two key halves, for long sequences); the launcher
+// says which runs when. Keys stream through LDS in blocks of 32 or 64 (K and
+// V both as [key][ch]). q, k and v come per (image, head) as [tpad][64]
 // matrices in fragment order (a wave's Q fragments are then 1 KB contiguous
-// loads). The blocks move from global memory straight into three
-// LDS buffers with DMA loads (buffer_load ... lds), two blocks ahead; each
-// 128-byte key row is stored with its 16-byte chunks XOR-swizzled by the
+// loads). The blocks move from global memory straight into LDS with DMA loads
+// (buffer_load ... lds), two blocks ahead or more; each 128-byte key row is
+// stored with its 16-byte chunks XOR-swizzled by the
 // row (swz below), so the row reads of K and the transpose reads of V hit
 // distinct banks.
 //
@@ -26,6 +29,8 @@
 // most rescales of O and, on the common path, the block max itself.
 // P is rounded to f16 for the PV product; the denominator keeps the fp32
 // weights (as in the reference, attention_online_f16_wmma_cf16.loom:195-216).
+#include <type_traits>
+
 #include "launch.hpp"
 
 namespace dhx {
@@ -61,6 +66,15 @@ __device__ __forceinline__ void vm_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// Calls f(integral_constant<int, I>) for I = 0 .. N-1.
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void for_constants(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        for_constants<N, I + 1>(f);
+    }
+}
+
 // The running softmax state of one lane's query (lane l holds query l % 32
 // and half of each 32-key sub-block's scores; see the top of this file).
 struct QueryState {
@@ -75,6 +89,44 @@ struct QueryState {
 __device__ __forceinline__ int tr_row_of(int lane) { return (lane & 15) >> 2; }
 __device__ __forceinline__ int tr_col_of(int lane) { return 16 * ((lane >> 4) & 1) + 4 * (lane & 3); }
 
+// This lane's element offsets inside a 32-key sub-block: of its four K
+// fragments, k(kk), and of its V transpose reads of 32-channel half ct, key
+// rows 4hi + tr_row and 8 further, v(ct, r) (the key rows 16 further have the
+// same swizzle). Computed once per kernel: the walks' steps are conditional,
+// and the compiler does not share address arithmetic between them.
+struct LaneOffsets {
+    int k_[4], v_[2][2];
+    __device__ __forceinline__ explicit LaneOffsets(int lane) {
+        const int l32 = lane & 31, hi = lane >> 5;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) k_[kk] = swz(l32, kk * 16 + hi * 8);
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) v_[ct][r] = swz(4 * hi + tr_row_of(lane) + 8 * r, ct * 32 + tr_col_of(lane));
+    }
+    __device__ __forceinline__ void step() {}
+    __device__ __forceinline__ int k(int kk) const { return k_[kk]; }
+    __device__ __forceinline__ int v(int ct, int r) const { return v_[ct][r]; }
+};
+
+// The same offsets from two registers instead of eight, for the kernel that
+// would not fit its 128 otherwise: the others differ from the first by one
+// exclusive or (chunk 2kk or 4ct, and a slot that changes in bit 1 with 8
+// rows), taken anew in every step.
+struct LaneOffsetsXor {
+    int k_, v_;
+    __device__ __forceinline__ explicit LaneOffsetsXor(int lane) {
+        const int l32 = lane & 31, hi = lane >> 5;
+        k_ = swz(l32, hi * 8);
+        v_ = swz(4 * hi + tr_row_of(lane), tr_col_of(lane));
+    }
+    // Keeps the compiler from computing the other offsets ahead of the steps.
+    __device__ __forceinline__ void step() { asm volatile("" : "+v"(k_), "+v"(v_)); }
+    __device__ __forceinline__ int k(int kk) const { return k_ ^ (kk << 4); }
+    __device__ __forceinline__ int v(int ct, int r) const { return (v_ ^ (ct << 5) ^ (r << 4)) + r * 8 * kHeadDim; }
+};
+
 // One sub-block of 32 keys (rows row0 .. row0+31 of the swizzled K and V
 // blocks in LDS, keys key0 .. key0+31 of the sequence of T):
 // S^T = K Q^T, masked past T, lazy running max, P = 2^(s log2e - m log2e),
@@ -83,27 +135,27 @@ __device__ __forceinline__ int tr_col_of(int lane) { return 16 * ((lane >> 4) & 
 // initial max of -1e30 would all overflow: its block max becomes the
 // running max directly, with one pass of exponentials instead of two (the
 // same values and rounding as the rescale path).
-template <bool FIRST = false>
+template <bool FIRST = false, class Offsets>
 __device__ __forceinline__ void attend32(QueryState& st, const half_t* sK, const half_t* sV, int row0, int key0,
-                                         int T, int lane) {
-    const int l32 = lane & 31, hi = lane >> 5;
+                                         int T, int lane, Offsets& at) {
+    at.step();
+    const int hi = lane >> 5;
     const float neg_inf = -__builtin_inff();
     float16_t s = {};
-    const int kr = row0 + l32;
+    sK += row0 * kHeadDim;
+    sV += row0 * kHeadDim;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) s = mfma32x32x16(*(const half8_t*)(sK + swz(kr, kk * 16 + hi * 8)), st.qf[kk], s);
+    for (int kk = 0; kk < 4; ++kk) s = mfma32x32x16(*(const half8_t*)(sK + at.k(kk)), st.qf[kk], s);
     // The V^T operands do not depend on the softmax: read them now so their
     // LDS latency hides under the exponentials. va[ct][ks] holds channel
     // ct*32 + l32 of keys key0 + 16ks + (j < 4 ? 4hi + j : 8 + 4hi + j - 4).
-    const int tr_row = tr_row_of(lane), tr_col = tr_col_of(lane);
     half8_t va[2][2];
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            const int vr = row0 + ks * 16 + 4 * hi + tr_row;
-            const half4_t a0 = lds_read_tr16(sV + swz(vr, ct * 32 + tr_col));
-            const half4_t a1 = lds_read_tr16(sV + swz(vr + 8, ct * 32 + tr_col));
+            const half4_t a0 = lds_read_tr16(sV + ks * 16 * kHeadDim + at.v(ct, 0));
+            const half4_t a1 = lds_read_tr16(sV + ks * 16 * kHeadDim + at.v(ct, 1));
             va[ct][ks] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     // s[r] is the score of key key0 + 8(r/4) + 4*hi + r%4 for query l32.
@@ -215,6 +267,18 @@ __device__ __forceinline__ int dma_lane_offset(int lane, int r0) {
 }
 __device__ __forceinline__ int dma_row_offset(int r0) { return (r0 >> 5) * 4096 + (r0 & 31) * 16; }
 
+// Buffer descriptors of one (image, head)'s q, k and v matrices.
+struct HeadSrc {
+    __amdgpu_buffer_rsrc_t q, k, v;
+    __device__ __forceinline__ HeadSrc(const AttentionArgs& p, int img, int head) {
+        const size_t mat = ((size_t)img * kHeads + head) * p.tpad * kHeadDim;
+        const int bytes = p.tpad * kHeadDim * 2;
+        q = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(p.q + mat), 0, bytes, kBufferRsrcWord3);
+        k = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(p.k + mat), 0, bytes, kBufferRsrcWord3);
+        v = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(p.v + mat), 0, bytes, kBufferRsrcWord3);
+    }
+};
+
 template <int NKB>
 __global__ __launch_bounds__(kThreads, 3) void attention_kernel(AttentionArgs p) {
     using KBT = KeyBlock<NKB>;
@@ -279,6 +343,7 @@ __global__ __launch_bounds__(kThreads, 3) void attention_kernel(AttentionArgs p)
         vm_barrier<0>();
     }
 
+    LaneOffsets at(lane);
     // Scores are s = (q / 8) . k: Q is scaled by 1/8 once (a power of two,
     // exact for normal f16 values), and the softmax weight of a score is
     // 2^(s*log2e - m*log2e), one FMA and one v_exp_f32.
@@ -294,9 +359,9 @@ __global__ __launch_bounds__(kThreads, 3) void attention_kernel(AttentionArgs p)
             const int key0 = kb * KBT::KB + sub * 32;
             if (key0 >= T) break;  // uniform across the workgroup
             if (NKB > 0 && kb == 0 && sub == 0)  // the unrolled walk: its first block is known at compile time
-                attend32<true>(st, sK, sV, 0, key0, T, lane);
+                attend32<true>(st, sK, sV, 0, key0, T, lane, at);
             else
-                attend32(st, sK, sV, sub * 32, key0, T, lane);
+                attend32(st, sK, sV, sub * 32, key0, T, lane, at);
         }
     };
     // Block kb is computed from buffer kb % 3 while the DMA of block kb+2
@@ -340,74 +405,180 @@ __global__ __launch_bounds__(kThreads, 3) void attention_kernel(AttentionArgs p)
     if (qrow < T) store_query(st, p.out, img * T + qb * QB + wave * 32, img * T + qrow, head, hi);
 }
 
-// Long sequences (512x512: 1029 tokens): each workgroup of 8 waves holds 128
-// queries as 4 query waves x 2 key halves. Half h walks key blocks
-// h*NH .. h*NH+NH-1 (32 keys each, NH known at compile time so the walk is
-// unrolled and every wait exact), streamed by its own 4 waves through its own
-// three DMA buffers; both halves meet at the same barriers. At the end the
-// second half's (running max, denominator, O^T) go through LDS to the first
-// half, which merges them (rescaling both to the larger max) and writes the
-// output. Twice the waves of attention_kernel for the same workgroups, so
-// the softmax VALU work of one wave overlaps the MFMAs and loads of others.
-constexpr int kSplitThreads = 512;
-constexpr int kSplitBlk = 32 * kHeadDim;  // halfs per 32-key K (or V) block
+// Short sequences in launches of at most one workgroup per CU: all N = ceil(T
+// / 32) key blocks are in flight from the start, each with LDS of its own
+// (8 KB per block), so a workgroup waits for one load latency instead of one
+// per block or two: one block 3.6 -> 3.0 us per launch, four 4.5 -> 3.8, five
+// 4.8 -> 4.2, six 5.2 -> 4.6 (HIP events, alone). At seven blocks (201 tokens)
+// the softmax chain of a wave, about 0.4 us per block, covers the loads in
+// attention_kernel already (5.34 -> 5.25 us, the forward unchanged). The Q
+// fragments come through LDS as well (4 KB per wave): with DMA loads only,
+// every wait is an exact count. The steps are those of attention_kernel, so a
+// query's result is bitwise the same.
+constexpr int kMaxResident = 6;
 
-// One key half's walk: blocks first .. first+NH-1 (past the sequence's last
-// block the DMA repeats that block and the compute is skipped), through the
-// half's own three K and three V buffers. The buffers are separate LDS
-// variables chosen at compile time (the caller branches on the half), so the
-// compiler can tell the buffer being read from the ones being filled and
-// adds no waits of its own for the DMA in flight.
-template <int NH>
-__device__ __forceinline__ void split_walk(QueryState& st, half_t* const (&kbuf)[3], half_t* const (&vbuf)[3],
-                                           const __amdgpu_buffer_rsrc_t& rk, const __amdgpu_buffer_rsrc_t& rv,
-                                           const half_t* qg, int first, int nkb, int qrow, bool active, int T,
-                                           int hwave, int lane) {
-    const int hi = lane >> 5;
-    const int voff = dma_lane_offset(lane, 8 * hwave), last = min(first + NH, nkb) - 1;
-    auto dma = [&](int buf, int s) {
-        const int kb = min(first + s, last), row = 8 * hwave, soff = dma_row_offset(kb * 32 + row);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)(kbuf[buf] + row * kHeadDim),
-                                                 16, voff, soff, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (__attribute__((address_space(3))) void*)(vbuf[buf] + row * kHeadDim),
-                                                 16, voff, soff, 0, 0);
-    };
-    // As in attention_kernel: block 0, the Q fragments, block 1; the first
-    // wait counts only block 1's two DMA loads.
-    dma(0, 0);
+// Halfs of a ring's or a resident set's i-th 32-key block out of N (a
+// placeholder past the last).
+template <int N>
+struct BlockLds {
+    template <int I>
+    static constexpr int at = I < N ? 32 * kHeadDim : 8;
+};
+
+template <int N>
+__device__ __forceinline__ void resident_walk(QueryState& st, half_t* const (&kbuf)[kMaxResident],
+                                              half_t* const (&vbuf)[kMaxResident], half_t* sq,
+                                              const __amdgpu_buffer_rsrc_t& rq, const __amdgpu_buffer_rsrc_t& rk,
+                                              const __amdgpu_buffer_rsrc_t& rv, int q0, int T, int wave, int lane) {
+    auto lds = [](half_t* a) { return (__attribute__((address_space(3))) void*)a; };
+    // The wave's 32 query rows (rows past T are tpad's padding: finite, and
+    // never stored), then its 8 rows of every key block.
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
-        st.qf[kk] = *(const half8_t*)(qg + frag_piece(min(qrow, T - 1), kk * 16 + hi * 8, kHeadDim));
-    asm volatile("" ::: "memory");
-    dma(1, 1);
-    vm_barrier<2>();
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, lds(sq + kk * 512), 16, lane * 16, (q0 / 32 * 4 + kk) * 1024, 0, 0);
+    const int row = wave * 8, voff = dma_lane_offset(lane, row);
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) st.qf[kk] *= (half_t)0.125f;
+    for (int kb = 0; kb < N; ++kb) {
+        const int soff = dma_row_offset(kb * 32 + row);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, lds(kbuf[kb] + row * kHeadDim), 16, voff, soff, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, lds(vbuf[kb] + row * kHeadDim), 16, voff, soff, 0, 0);
+    }
     st.o[0] = st.o[1] = float16_t{};
-    // Step s: block first+s from buffer s % 3 while block s+2's DMA fills
-    // buffer (s+2) % 3 (released by the previous barrier); the barrier
-    // leaves only that DMA in flight, so block s+1 has landed for every wave.
+    LaneOffsets at(lane);
+    const bool active = q0 < T;  // waves whose queries all lie past T only move K and V
+    for_constants<N>([&](auto KB) {
+        constexpr int kb = decltype(KB)::value;
+        if constexpr (kb == 0) {
+            vm_barrier<2 * N - 1>();  // Q has landed (and the first K block)
 #pragma unroll
-    for (int s = 0; s < NH; ++s) {
-        if (s + 2 < NH) dma((s + 2) % 3, s + 2);
-        const int kb = first + s;
-        if (active && kb < nkb) {
-            if (s == 0)
-                attend32<true>(st, kbuf[0], vbuf[0], 0, kb * 32, T, lane);
-            else
-                attend32(st, kbuf[s % 3], vbuf[s % 3], 0, kb * 32, T, lane);
+            for (int kk = 0; kk < 4; ++kk) st.qf[kk] = *(const half8_t*)(sq + kk * 512 + lane * 8) * (half_t)0.125f;
         }
-        if (s + 2 < NH)
-            vm_barrier<2>();
+        vm_barrier<2 * (N - 1 - kb)>();  // only later blocks may be outstanding
+        if (active) attend32<kb == 0>(st, kbuf[kb], vbuf[kb], 0, kb * 32, T, lane, at);
+    });
+}
+
+template <int N>
+__global__ __launch_bounds__(kThreads, 2) void attention_resident_kernel(AttentionArgs p) {
+    using L = BlockLds<N>;
+    __shared__ __attribute__((aligned(16))) half_t k0[L::template at<0>], k1[L::template at<1>], k2[L::template at<2>], k3[L::template at<3>], k4[L::template at<4>], k5[L::template at<5>];
+    __shared__ __attribute__((aligned(16))) half_t v0[L::template at<0>], v1[L::template at<1>], v2[L::template at<2>], v3[L::template at<3>], v4[L::template at<4>], v5[L::template at<5>];
+    __shared__ __attribute__((aligned(16))) half_t sq[4 * 4 * 512];  // four fragments per wave
+    const int nqb = (p.tokens + QB - 1) / QB, total = nqb * kHeads * p.images;
+    const int per = (total + 7) >> 3, g = blockIdx.x, t = (g & 7) * per + (g >> 3);
+    if ((g >> 3) >= per || t >= total) return;  // uniform per workgroup
+    const int qb = t % nqb, head = (t / nqb) % kHeads, img = t / (nqb * kHeads);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q0 = qb * QB + wave * 32, q = q0 + (lane & 31);
+    const HeadSrc src(p, img, head);
+    half_t* const kbuf[kMaxResident] = {k0, k1, k2, k3, k4, k5};
+    half_t* const vbuf[kMaxResident] = {v0, v1, v2, v3, v4, v5};
+    QueryState st;
+    resident_walk<N>(st, kbuf, vbuf, sq + wave * 2048, src.q, src.k, src.v, q0, p.tokens, wave, lane);
+    if (q < p.tokens) store_query(st, p.out, img * p.tokens + q0, img * p.tokens + q, head, lane >> 5);
+}
+
+// Long sequences: workgroups of 2 QW waves hold 32 QW queries as QW query
+// waves x 2 key halves. Half h walks key blocks h*nh .. h*nh+nh-1 (32 keys
+// each, nh = ceil(blocks / 2)) through its own three K and three V buffers;
+// both halves meet at the same barriers. At the end the second half's
+// (running max, denominator, O^T) go through LDS to the first half, which
+// merges them (rescaling both to the larger max) and writes the output. What
+// bounds it is the wave's own chain of score MFMAs, about 85 vector
+// instructions (16 of them exponentials) and PV MFMAs, some 700 - 850 cycles
+// per 32 keys, MFMA and vector issue hardly overlapping: two waves per SIMD
+// take the time of one twice, so a launch is as fast as its keys per SIMD are
+// few. Halves and 64-query workgroups spread them (512x512 batch 1: 54
+// workgroups of 8 waves -> 102 of 4, 13.1 -> 10.6 us); deeper rings did not
+// help (four to eight buffers per half: 13.1 -> 13.3 - 14.3 us).
+constexpr int kSplitBlk = 32 * kHeadDim;  // halfs per 32-key K (or V) block
+
+// One key half's walk from block `first` on (past the sequence's last block
+// the DMA repeats that block and the compute is skipped). The buffers are
+// separate LDS variables chosen at compile time (the caller branches on the
+// half), so the compiler can tell the buffer being read from the ones being
+// filled and adds no waits of its own for the DMA in flight. The Q fragments
+// come through LDS too (sq, 4 KB, one of the third buffers): with DMA loads
+// only, every wait is an exact count. NH > 0: nh = NH, unrolled.
+template <int NH, int QW>
+__device__ __forceinline__ void split_walk(QueryState& st, half_t* const (&kbuf)[3], half_t* const (&vbuf)[3],
+                                           const HeadSrc& src, half_t* sq, int first, int nh_rt, int nkb, int q0, int T,
+                                           int hwave, int lane) {
+    constexpr int LOADS = 4 / QW;  // 8-row DMA loads per matrix, wave and block
+    const int nh = NH > 0 ? NH : nh_rt, last = min(first + nh, nkb) - 1;
+    int voff[4];  // sized 4, not LOADS (see attention_kernel)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) voff[i] = dma_lane_offset(lane, 8 * (hwave * LOADS + i));
+    auto lds = [](half_t* a) { return (__attribute__((address_space(3))) void*)a; };
+    auto dma = [&](int buf, int s) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int row = 8 * (hwave * LOADS + i), soff = dma_row_offset(min(first + s, last) * 32 + row);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(src.k, lds(kbuf[buf] + row * kHeadDim), 16, voff[i], soff, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(src.v, lds(vbuf[buf] + row * kHeadDim), 16, voff[i], soff, 0, 0);
+        }
+    };
+    constexpr int kPerBlock = 2 * LOADS;
+    // Query rows past T are tpad's padding: finite, and never stored. Each
+    // wave takes its fragments before the barrier after which sq is filled
+    // with a block.
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src.q, lds(sq + kk * 512), 16, lane * 16, (q0 / 32 * 4 + kk) * 1024, 0, 0);
+    dma(0, 0);
+    dma(1, 1);
+    st.o[0] = st.o[1] = float16_t{};
+    std::conditional_t<NH == 0 && QW == 4, LaneOffsetsXor, LaneOffsets> at(lane);
+    const bool active = q0 < T;  // waves whose queries all lie past T only move K and V
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPerBlock) : "memory");
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) st.qf[kk] = *(const half8_t*)(sq + kk * 512 + lane * 8) * (half_t)0.125f;
+    vm_barrier<kPerBlock>();
+    // Step s: block first+s from buffer s % 3 while block s+2's DMA fills
+    // the buffer that the previous barrier released; the barrier leaves only
+    // that DMA in flight, so block s+1 has landed for every wave.
+    auto attend = [&](int b, int s, bool first_block) {
+        const int kb = first + s;
+        if (!active || kb >= nkb) return;
+        if (first_block)
+            attend32<true>(st, kbuf[b], vbuf[b], 0, kb * 32, T, lane, at);
         else
-            vm_barrier<0>();
+            attend32(st, kbuf[b], vbuf[b], 0, kb * 32, T, lane, at);
+    };
+    if constexpr (NH > 0) {
+#pragma unroll
+        for (int s = 0; s < NH; ++s) {
+            if (s + 2 < NH) dma((s + 2) % 3, s + 2);
+            attend(s % 3, s, s == 0);
+            if (s + 2 < NH)
+                vm_barrier<kPerBlock>();
+            else
+                vm_barrier<0>();
+        }
+    } else {
+        // As in attention_kernel: every step issues its DMA (past the last
+        // block it repeats it) and waits the same way; the repeats are drained
+        // at the end.
+        auto step = [&](int b, int s) {
+            dma((b + 2) % 3, s + 2);
+            attend(b, s, false);
+            vm_barrier<kPerBlock>();
+        };
+        for (int s = 0; s < nh; s += 3) {
+            step(0, s);
+            if (s + 1 >= nh) break;
+            step(1, s + 1);
+            if (s + 2 >= nh) break;
+            step(2, s + 2);
+        }
+        vm_barrier<0>();
     }
 }
 
-// Two workgroups per CU: four waves per SIMD (the bound below), which caps
-// the kernel at 128 VGPRs; one register more halves the resident workgroups.
-template <int NH>
-__global__ __launch_bounds__(kSplitThreads, 4) void attention_split_kernel(AttentionArgs p) {
+// QW = 4: two workgroups per CU, four waves per SIMD, which caps the kernel
+// at 128 VGPRs; one register more halves the resident workgroups.
+template <int NH, int QW>
+__global__ __launch_bounds__(2 * QW * kWave, QW == 4 ? 4 : 2) void attention_split_kernel(AttentionArgs p) {
     // Per half three K and three V blocks of 4 KB (48 KB), as separate
     // variables (the compiler tells distinct variables apart, not the rows of
     // one array); reused at the end for the merge.
@@ -415,42 +586,39 @@ __global__ __launch_bounds__(kSplitThreads, 4) void attention_split_kernel(Atten
     __shared__ __attribute__((aligned(16))) half_t v00[kSplitBlk], v01[kSplitBlk], v02[kSplitBlk];
     __shared__ __attribute__((aligned(16))) half_t k10[kSplitBlk], k11[kSplitBlk], k12[kSplitBlk];
     __shared__ __attribute__((aligned(16))) half_t v10[kSplitBlk], v11[kSplitBlk], v12[kSplitBlk];
-    const int nqb = (p.tokens + QB - 1) / QB, total = nqb * kHeads * p.images;
+    constexpr int Q = 32 * QW;  // queries per workgroup
+    const int nqb = (p.tokens + Q - 1) / Q, total = nqb * kHeads * p.images;
     const int per = (total + 7) >> 3, g = blockIdx.x, t = (g & 7) * per + (g >> 3);
     if ((g >> 3) >= per || t >= total) return;  // uniform per workgroup
     const int qb = t % nqb, head = (t / nqb) % kHeads, img = t / (nqb * kHeads);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int qw = wave & 3, half = wave >> 2;  // query wave; key half (uniform per wave)
+    const int qw = wave % QW, half = wave / QW;  // query wave; key half (uniform per wave)
     const int l32 = lane & 31, hi = lane >> 5;
-    const int T = p.tokens, nkb = (T + 31) / 32;  // nkb <= 2 * NH and nkb * 32 <= tpad (launcher checks)
-    const size_t bh = (size_t)img * kHeads + head;
-    const uint32_t bytes = (uint32_t)p.tpad * kHeadDim * 2;
-    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<half_t*>(p.k + bh * p.tpad * kHeadDim), 0, bytes, kBufferRsrcWord3);
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<half_t*>(p.v + bh * p.tpad * kHeadDim), 0, bytes, kBufferRsrcWord3);
-    const half_t* qg = p.q + bh * p.tpad * kHeadDim;
-    const int qrow = qb * QB + qw * 32 + l32;
-    const bool active = qb * QB + qw * 32 < T;  // waves whose queries all lie past T only move K and V
+    const int T = p.tokens, nkb = (T + 31) / 32;  // nkb <= 2 * nh and nkb * 32 <= tpad
+    const int nh = NH > 0 ? NH : (nkb + 1) / 2;
+    const HeadSrc src(p, img, head);
+    const int q0 = qb * Q + qw * 32, qrow = q0 + l32;
+    // Query wave qw's Q fragments (both halves' waves load the same).
+    half_t* const sq = qw == 0 ? k02 : qw == 1 ? v02 : qw == 2 ? k12 : v12;
     QueryState st;
     if (half == 0) {
         half_t* const kb[3] = {k00, k01, k02};
         half_t* const vb[3] = {v00, v01, v02};
-        split_walk<NH>(st, kb, vb, rk, rv, qg, 0, nkb, qrow, active, T, qw, lane);
+        split_walk<NH, QW>(st, kb, vb, src, sq, 0, nh, nkb, q0, T, qw, lane);
     } else {
         half_t* const kb[3] = {k10, k11, k12};
         half_t* const vb[3] = {v10, v11, v12};
-        split_walk<NH>(st, kb, vb, rk, rv, qg, NH, nkb, qrow, active, T, qw, lane);
+        split_walk<NH, QW>(st, kb, vb, src, sq, nh, nh, nkb, q0, T, qw, lane);
     }
     // Merge: the second half hands its 34 values per lane (max, denominator,
     // O^T) to the first through LDS; both are rescaled to the larger max.
     // Every wave passed the walk's last barrier, which waited for all of its
     // DMA loads, so the buffers are free. Value f of query wave qw sits in
-    // buffer f / 4 at [(f % 4) * 4 + qw][lane] (f is a constant, so each
+    // buffer f / 4 at [(f % 4) * QW + qw][lane] (f is a constant, so each
     // access names its buffer).
     half_t* const bufs[12] = {k00, k01, k02, v00, v01, v02, k10, k11, k12, v10, v11, v12};
     auto slot = [&](int f) -> float* {
-        return reinterpret_cast<float*>(bufs[f / 4]) + ((f % 4) * 4 + qw) * 64 + lane;
+        return reinterpret_cast<float*>(bufs[f / 4]) + ((f % 4) * QW + qw) * 64 + lane;
     };
     if (half == 1) {
         *slot(0) = st.m_run;
@@ -465,31 +633,64 @@ __global__ __launch_bounds__(kSplitThreads, 4) void attention_split_kernel(Atten
     if (half == 1 || qrow >= T) return;
     const float m1 = *slot(0), m = fmaxf(st.m_run, m1);
     const float a0 = fast_exp2((st.m_run - m) * kLog2e), a1 = fast_exp2((m1 - m) * kLog2e);
-    st.l_run = st.l_run * a0 + *slot(1) * a1;
+    st.l_run = fmaf(st.l_run, a0, *slot(1) * a1);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        st.o[0][r] = st.o[0][r] * a0 + *slot(2 + r) * a1;
-        st.o[1][r] = st.o[1][r] * a0 + *slot(18 + r) * a1;
+        st.o[0][r] = fmaf(st.o[0][r], a0, *slot(2 + r) * a1);
+        st.o[1][r] = fmaf(st.o[1][r], a0, *slot(18 + r) * a1);
     }
-    store_query(st, p.out, img * T + qb * QB + qw * 32, img * T + qrow, head, hi);
+    store_query(st, p.out, img * T + q0, img * T + qrow, head, hi);
+}
+
+// The longest sequences attention_kernel takes: from here on the keys are
+// walked in two halves (attention_split_kernel). The walk is part of a result's
+// arithmetic, so it depends on the sequence only, not on the launch.
+constexpr int kSplitBlocks = 16;  // blocks of 32 keys, from 481 tokens on
+constexpr int kRound = 256;       // workgroups of one per CU
+
+template <int N>
+hipError_t launch_resident(const AttentionArgs& a, int nkb, dim3 grid, hipStream_t s) {
+    if constexpr (N > 1)
+        if (nkb < N) return launch_resident<N - 1>(a, nkb, grid, s);
+    hipLaunchKernelGGL(attention_resident_kernel<N>, grid, dim3(kThreads), 0, s, a);
+    return hipGetLastError();
+}
+
+template <int NH, int QW>
+hipError_t launch_split(const AttentionArgs& a, int groups, hipStream_t s) {
+    hipLaunchKernelGGL((attention_split_kernel<NH, QW>), dim3((groups + 7) & ~7), dim3(2 * QW * kWave), 0, s, a);
+    return hipGetLastError();
 }
 
 }  // namespace
 
+// 224x224 (201 tokens): seven blocks of 32 keys, unrolled. Fewer blocks in
+// launches of at most one workgroup per CU: all resident. From 481 tokens on
+// two key halves, on workgroups of 64 queries where one round of them covers
+// the launch, which then runs on twice the CUs with one wave per SIMD (whole
+// forward, 128 -> 64 queries: 384x384 batch 3 439 -> 421 us, 512x512 batch 1
+// 455 -> 424, 720x720 batch 1 620 -> 569; attention_kernel with its run-time
+// count before: 443, -, 666), else of 128 (1024x1024 batch 2 1852 -> 1800;
+// equal to attention_kernel from 581 tokens on, 5 % slower at 405). 512x512
+// (17 blocks per half) in more than one round takes the unrolled walk (batch 8
+// 975 -> 964 us); in one round its 80 KB of code cost more to fetch than they
+// save (batch 1 449 against 424, batch 4 636 against 629). Otherwise blocks of
+// 64 keys with a run-time count.
 hipError_t launch_attention(const AttentionArgs& a, hipStream_t s) {
-    const int total = (a.tokens + QB - 1) / QB * kHeads * a.images;
+    const int nqb = (a.tokens + QB - 1) / QB, total = nqb * kHeads * a.images;
+    const int total64 = (a.tokens + 63) / 64 * kHeads * a.images;
     const dim3 grid((total + 7) & ~7), block(kThreads);
-    // 224x224 (201 tokens): seven blocks of 32 keys, unrolled. 512x512 (1029
-    // tokens, 33 blocks of 32): the split-key kernel with 17 blocks per half.
-    // Otherwise blocks of 64 with a run-time count.
-    const int nkb32 = (a.tokens + 31) / 32;
-    if (nkb32 == 7) {
-        hipLaunchKernelGGL(attention_kernel<7>, grid, block, 0, s, a);
-    } else if ((nkb32 + 1) / 2 == 17 && nkb32 * 32 <= a.tpad) {
-        hipLaunchKernelGGL(attention_split_kernel<17>, grid, dim3(kSplitThreads), 0, s, a);
-    } else {
-        hipLaunchKernelGGL(attention_kernel<0>, grid, block, 0, s, a);
+    const int nkb = (a.tokens + 31) / 32;
+    if (nkb <= kMaxResident && total <= kRound) return launch_resident<kMaxResident>(a, nkb, grid, s);
+    if (nkb >= kSplitBlocks) {
+        if (total64 <= kRound) return launch_split<0, 2>(a, total64, s);
+        if ((nkb + 1) / 2 == 17 && total > kRound) return launch_split<17, 4>(a, total, s);
+        return launch_split<0, 4>(a, total, s);
     }
+    if (nkb == 7)
+        hipLaunchKernelGGL(attention_kernel<7>, grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL(attention_kernel<0>, grid, block, 0, s, a);
     return hipGetLastError();
 }
 

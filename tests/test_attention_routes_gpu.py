@@ -1,0 +1,62 @@
+"""Every attention kernel a sequence can run on gives an image the same bits:
+launches on both sides of each rule's edge (one workgroup per CU for the
+resident and the 64-query kernels, one round for the unrolled walk) against
+one larger launch of the same images, and the sequences around the edge of the
+two-halves walk against the float64 oracle."""
+import numpy as np
+import pytest
+
+import oracle
+
+from test_kernels_gpu import K_ATTN, allocf, check, eng, f16, heads_frag, readf, run, up  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def launch(e, mats, images, grid):
+    T = grid * grid + 5
+    tpad = (T + 127) // 128 * 128
+    ins = [up(e, heads_frag(m[:images * T], images, T, tpad)) for m in mats]
+    out = allocf(e, images * T, 384)
+    run(e, K_ATTN, [images, grid, tpad], ins + [out])
+    return readf(e, out, images * T, 384)
+
+
+def inputs(grid, images, scale=2.0):
+    rng = np.random.default_rng(grid)
+    rows = images * (grid * grid + 5)
+    return [f16(rng.normal(size=(rows, 384)) * s) for s in (scale, 1.0, 1.0)]
+
+
+# (grid, images of the large launch, images of the others): 1, 3, 5 and 6 key
+# blocks (resident up to 256 workgroups), 16 and 19 blocks (64-query
+# workgroups up to 256 of them), 1029 tokens (64 queries to 2 images, 128 from
+# 3, the unrolled walk from 5), 2030 tokens.
+ROUTES = [(4, 50, (1, 42, 43)), (8, 50, (1, 42, 43)), (12, 24, (1, 21, 22)), (13, 24, (1, 21, 22)),
+          (22, 8, (1, 5, 6)), (24, 8, (1, 4, 5)), (32, 6, (1, 2, 3, 4, 5)), (45, 3, (1, 2))]
+
+
+@pytest.mark.parametrize("grid,most,counts", ROUTES)
+def test_images_do_not_depend_on_the_launch(eng, grid, most, counts):  # noqa: F811
+    mats = inputs(grid, most)
+    T = grid * grid + 5
+    want = launch(eng, mats, most, grid)
+    assert np.all(np.isfinite(want))
+    for images in counts:
+        got = launch(eng, mats, images, grid)
+        assert np.array_equal(got, want[:images * T]), images
+
+
+@pytest.mark.parametrize("grid", [1, 5, 7, 21, 22, 25])
+@pytest.mark.parametrize("scale", [0.0, 4.0])
+def test_edges_match_the_oracle(eng, grid, scale):  # noqa: F811
+    # P is rounded to f16 (2^-11 relative) before a product whose weights sum
+    # to one, and the output to f16: 2^-9 max|V| bounds both, as in the
+    # per-kernel attention test.
+    q, k, v = inputs(grid, 2, scale)
+    T = grid * grid + 5
+    got = launch(eng, [q, k, v], 2, grid)
+    for i in range(2):
+        rows = slice(i * T, (i + 1) * T)
+        want = oracle.attention(*(m[rows].astype(np.float64) for m in (q, k, v)))
+        check(got[rows], want, atol=2.0**-9 * np.abs(v[rows].astype(np.float64)).max(), what=f"T={T} image {i}")
