@@ -48,6 +48,7 @@ using SplitTile = Tile<128, 128, 4, 1>;
 using ResidRing32 = Tile<32, 64, 1, 2, 128>;
 using ResidRing64 = Tile<64, 64, 2, 2, 64>;
 using ResidRing128 = Tile<128, 64, 4, 2, 64>;
+using ResidRing128W = Tile<128, 128, 4, 2, 64>;
 using SwigluRing64 = Tile<64, 128, 2, 2, 32>;
 using SwigluRing128 = Tile<128, 128, 4, 2, 32>;
 using SwigluRing128W = Tile<128, 192, 4, 3, 32>;
@@ -121,14 +122,21 @@ hipError_t launch_resid(const ResidArgs& a, hipStream_t s) {
     // Beside another image group's kernels (a.shared) the 128x64 ring, which
     // takes a CU's LDS whole, loses to the tiles below (705 -> 742 us at 2 x
     // 3216 rows).
+    // One more size for the down projection, 128x128 tiles to 10880 rows: 6432
+    // rows 736 -> 699 us, 8643 rows 886 -> 858, 8232 rows 1029 -> 1008 (one
+    // chain); beside another group 705 -> 733 at 2 x 6432 rows. The o-projection,
+    // with three stages to a tile, gains nothing from it.
     const int round = a.rows <= kRound / 6 * 32   ? 32
                       : a.rows <= kRound / 6 * 64 ? 64
-                      : a.rows <= kRound / 6 * 128 && !a.shared ? 128 : 0;
+                      : a.shared                  ? 0
+                      : a.rows <= kRound / 6 * 128 ? 128
+                      : a.rows <= kRound / 3 * 128 ? 256 : 0;
     if (a.k == kHidden && round == 32) return launch_resid_ring<ResidRing32, 4, kHidden>(a, s);
     if (a.k == kHidden && round == 64) return launch_resid_ring<ResidRing64, 5, kHidden>(a, s);
     if (a.k == kHidden && round == 128) return launch_resid_ring<ResidRing128, 4, kHidden>(a, s);
     if (a.k == kFF && (round == 32 || round == 64)) return launch_resid_ring<ResidRing64, 5, kFF>(a, s);
     if (a.k == kFF && round == 128) return launch_resid_ring<ResidRing128, 4, kFF>(a, s);
+    if (a.k == kFF && round == 256) return launch_resid_ring<ResidRing128W, 4, kFF>(a, s);
     // The K loop walks its stages six at a time (gemm_main_dma).
     if (a.k % (6 * ResidTile::BK) != 0) return hipErrorInvalidValue;
     if (a.k == kHidden) {  // the o-projection: three 128-deep stages, unrolled

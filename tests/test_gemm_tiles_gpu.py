@@ -28,7 +28,7 @@ def run(e, kernel, scalars, bindings, beside=None):
 @pytest.mark.parametrize("kdim", [384, 1536])
 def test_resid_rows_do_not_depend_on_the_tile(eng, kdim):  # noqa: F811
     rng = np.random.default_rng(kdim)
-    most = 6000
+    most = 11000
     a, x0 = f16(rng.normal(size=(most, kdim))), f16(rng.normal(size=(most, 384)) * 2 + 0.5)
     w = upf(eng, f16(rng.normal(size=(384, kdim)) * 0.03))
     b = up(eng, (rng.normal(size=384) * 0.1).astype(np.float32))
@@ -46,7 +46,7 @@ def test_resid_rows_do_not_depend_on_the_tile(eng, kdim):  # noqa: F811
         return y, eng.read(st, np.float32, (rows, 12))
 
     want, want_stats = launch(most)
-    for rows in (1, 32, 33, 65, 1344, 1345, 2688, 2689, 5376, 5377):
+    for rows in (1, 32, 33, 65, 1344, 1345, 2688, 2689, 5376, 5377, 10880, 10881):
         for beside in (False, True):
             got, stats = launch(rows, beside)
             assert np.array_equal(got, want[:rows]), (rows, beside)
