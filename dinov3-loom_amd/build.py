@@ -41,7 +41,9 @@ ARCH = "gfx950"
 # Packed-FP32 instructions stay off in device code (hipcc forms them from
 # plain float code otherwise); the host pass warns that it does not know the
 # feature, which is harmless.
-DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# The first kernel arguments arrive in scalar registers (kernels/launch.hpp).
+DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-I", os.path.join(ROOT, "include"),
           "-Wall", "-Wno-unused-function"]
 

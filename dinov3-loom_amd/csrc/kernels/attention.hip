@@ -280,7 +280,8 @@ struct HeadSrc {
 };
 
 template <int NKB>
-__global__ __launch_bounds__(kThreads, 3) void attention_kernel(AttentionArgs p) {
+__global__ __launch_bounds__(kThreads, 3) void attention_kernel(DHX_ATTENTION_PARAMS) {
+    const AttentionArgs p{q_, k_, v_, out_, images_, tokens_, tpad_};
     using KBT = KeyBlock<NKB>;
     __shared__ __attribute__((aligned(16))) half_t sK0[KBT::BLK], sK1[KBT::BLK], sK2[KBT::BLK];
     __shared__ __attribute__((aligned(16))) half_t sV0[KBT::BLK], sV1[KBT::BLK], sV2[KBT::BLK];
@@ -459,7 +460,8 @@ __device__ __forceinline__ void resident_walk(QueryState& st, half_t* const (&kb
 }
 
 template <int N>
-__global__ __launch_bounds__(kThreads, 2) void attention_resident_kernel(AttentionArgs p) {
+__global__ __launch_bounds__(kThreads, 2) void attention_resident_kernel(DHX_ATTENTION_PARAMS) {
+    const AttentionArgs p{q_, k_, v_, out_, images_, tokens_, tpad_};
     using L = BlockLds<N>;
     __shared__ __attribute__((aligned(16))) half_t k0[L::template at<0>], k1[L::template at<1>], k2[L::template at<2>], k3[L::template at<3>], k4[L::template at<4>], k5[L::template at<5>];
     __shared__ __attribute__((aligned(16))) half_t v0[L::template at<0>], v1[L::template at<1>], v2[L::template at<2>], v3[L::template at<3>], v4[L::template at<4>], v5[L::template at<5>];
@@ -578,7 +580,8 @@ __device__ __forceinline__ void split_walk(QueryState& st, half_t* const (&kbuf)
 // QW = 4: two workgroups per CU, four waves per SIMD, which caps the kernel
 // at 128 VGPRs; one register more halves the resident workgroups.
 template <int NH, int QW>
-__global__ __launch_bounds__(2 * QW * kWave, QW == 4 ? 4 : 2) void attention_split_kernel(AttentionArgs p) {
+__global__ __launch_bounds__(2 * QW * kWave, QW == 4 ? 4 : 2) void attention_split_kernel(DHX_ATTENTION_PARAMS) {
+    const AttentionArgs p{q_, k_, v_, out_, images_, tokens_, tpad_};
     // Per half three K and three V blocks of 4 KB (48 KB), as separate
     // variables (the compiler tells distinct variables apart, not the rows of
     // one array); reused at the end for the merge.
@@ -652,14 +655,12 @@ template <int N>
 hipError_t launch_resident(const AttentionArgs& a, int nkb, dim3 grid, hipStream_t s) {
     if constexpr (N > 1)
         if (nkb < N) return launch_resident<N - 1>(a, nkb, grid, s);
-    hipLaunchKernelGGL(attention_resident_kernel<N>, grid, dim3(kThreads), 0, s, a);
-    return hipGetLastError();
+    return start(attention_resident_kernel<N>, grid, dim3(kThreads), 0, s, a);
 }
 
 template <int NH, int QW>
 hipError_t launch_split(const AttentionArgs& a, int groups, hipStream_t s) {
-    hipLaunchKernelGGL((attention_split_kernel<NH, QW>), dim3((groups + 7) & ~7), dim3(2 * QW * kWave), 0, s, a);
-    return hipGetLastError();
+    return start(attention_split_kernel<NH, QW>, dim3((groups + 7) & ~7), dim3(2 * QW * kWave), 0, s, a);
 }
 
 }  // namespace
@@ -687,11 +688,7 @@ hipError_t launch_attention(const AttentionArgs& a, hipStream_t s) {
         if ((nkb + 1) / 2 == 17 && total > kRound) return launch_split<17, 4>(a, total, s);
         return launch_split<0, 4>(a, total, s);
     }
-    if (nkb == 7)
-        hipLaunchKernelGGL(attention_kernel<7>, grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL(attention_kernel<0>, grid, block, 0, s, a);
-    return hipGetLastError();
+    return nkb == 7 ? start(attention_kernel<7>, grid, block, 0, s, a) : start(attention_kernel<0>, grid, block, 0, s, a);
 }
 
 }  // namespace dhx

@@ -57,10 +57,9 @@ using QkvRing64W = Tile<64, 128, 2, 2, 64>;
 using QkvRing128 = Tile<128, 128, 4, 2, 64>;
 constexpr int kRound = 256;  // workgroups of one per CU
 
-template <class T, class Args>
-hipError_t launch(void (*kernel)(Args), int tiles, const Args& a, hipStream_t s) {
-    hipLaunchKernelGGL(kernel, dim3(gemm::tile_grid(tiles)), dim3(T::THREADS), 0, s, a);
-    return hipGetLastError();
+template <class T, class Kernel, class Args>
+hipError_t launch(Kernel kernel, int tiles, const Args& a, hipStream_t s) {
+    return start(kernel, dim3(gemm::tile_grid(tiles)), dim3(T::THREADS), 0, s, a);
 }
 
 }  // namespace
@@ -76,18 +75,16 @@ static hipError_t launch_qkv_tiles(const QkvArgs& a, hipStream_t s) {
     const int tiles = tiles_for<T>(a.images * (a.grid * a.grid + kPrefix), 3 * kHidden);
     const dim3 grid(gemm::tile_grid(tiles));
     const size_t lds = gemm::rope_lds_bytes(a.grid);
-    if (a.stats) hipLaunchKernelGGL((gemm::qkv_rope_kernel<T, true>), grid, dim3(T::THREADS), lds, s, a);
-    else hipLaunchKernelGGL((gemm::qkv_rope_kernel<T, false>), grid, dim3(T::THREADS), lds, s, a);
-    return hipGetLastError();
+    return a.stats ? start(gemm::qkv_rope_kernel<T, true>, grid, dim3(T::THREADS), lds, s, a)
+                   : start(gemm::qkv_rope_kernel<T, false>, grid, dim3(T::THREADS), lds, s, a);
 }
 
 template <class T, int NST>
 static hipError_t launch_qkv_ring(const QkvArgs& a, hipStream_t s) {
     const dim3 grid(gemm::tile_grid(tiles_for<T>(a.images * (a.grid * a.grid + kPrefix), 3 * kHidden)));
     const size_t lds = gemm::rope_lds_bytes(a.grid);
-    if (a.stats) hipLaunchKernelGGL((gemm::qkv_ring_kernel<T, NST, true>), grid, dim3(T::THREADS), lds, s, a);
-    else hipLaunchKernelGGL((gemm::qkv_ring_kernel<T, NST, false>), grid, dim3(T::THREADS), lds, s, a);
-    return hipGetLastError();
+    return a.stats ? start(gemm::qkv_ring_kernel<T, NST, true>, grid, dim3(T::THREADS), lds, s, a)
+                   : start(gemm::qkv_ring_kernel<T, NST, false>, grid, dim3(T::THREADS), lds, s, a);
 }
 
 // As for the residual GEMMs: the smallest ring tile that one round of
@@ -163,17 +160,15 @@ template <class T, int NS>
 static hipError_t launch_swiglu_tiles(const SwigluArgs& a, hipStream_t s) {
     static_assert(kHidden % (6 * T::BK) == 0, "the K loop walks its stages six at a time");
     const int grid = gemm::tile_grid_split<NS>((a.rows + T::BM - 1) / T::BM, 2 * kFF / T::BN);
-    if (a.stats) hipLaunchKernelGGL((gemm::swiglu_kernel<T, true, NS>), dim3(grid), dim3(T::THREADS), 0, s, a);
-    else hipLaunchKernelGGL((gemm::swiglu_kernel<T, false, NS>), dim3(grid), dim3(T::THREADS), 0, s, a);
-    return hipGetLastError();
+    return a.stats ? start(gemm::swiglu_kernel<T, true, NS>, dim3(grid), dim3(T::THREADS), 0, s, a)
+                   : start(gemm::swiglu_kernel<T, false, NS>, dim3(grid), dim3(T::THREADS), 0, s, a);
 }
 
 template <class T, int NST>
 static hipError_t launch_swiglu_ring(const SwigluArgs& a, hipStream_t s) {
     const dim3 grid(gemm::tile_grid(tiles_for<T>(a.rows, 2 * kFF)));
-    if (a.stats) hipLaunchKernelGGL((gemm::swiglu_ring_kernel<T, NST, true>), grid, dim3(T::THREADS), 0, s, a);
-    else hipLaunchKernelGGL((gemm::swiglu_ring_kernel<T, NST, false>), grid, dim3(T::THREADS), 0, s, a);
-    return hipGetLastError();
+    return a.stats ? start(gemm::swiglu_ring_kernel<T, NST, true>, grid, dim3(T::THREADS), 0, s, a)
+                   : start(gemm::swiglu_ring_kernel<T, NST, false>, grid, dim3(T::THREADS), 0, s, a);
 }
 
 // As for the residual GEMMs: the smallest ring tile that one round of

@@ -74,7 +74,8 @@ __device__ __forceinline__ void pair_stats(float* stats, size_t m, int slot, con
 // wave rounds its 32 x 64 block to f16 into LDS, then writes it as fragment
 // pieces, lane (l, hi) taking row l and the half hi of each 16-column block.
 template <class T, bool STATS>
-__global__ __launch_bounds__(T::THREADS) void patch_embed_kernel(PatchEmbedArgs p) {
+__global__ __launch_bounds__(T::THREADS) void patch_embed_kernel(DHX_PATCH_PARAMS) {
+    const PatchEmbedArgs p{pixels_, w_, bias_, prefix_, x_, images_, grid_, prefix_stats_, stats_};
     static_assert(T::TN == 64 && T::TM == 32, "one 32-row block and one statistics slot per wave");
     constexpr int SP = T::TN + 8;  // staging pitch in halfs
     static_assert(T::WAVES * T::TM * SP <= T::LDS_HALFS, "staging fits the stage buffers");
@@ -186,7 +187,14 @@ __device__ __forceinline__ void qkv_epilogue(const QkvArgs& p, const Acc<T>& acc
                                              const float* bias, const float* wsum, const float* rope_lds, Norm&& norm) {
     const int P = p.grid * p.grid, Tok = P + kPrefix, M = p.images * Tok;
     const int part = f.n_base / kHidden, head0 = (f.n_base % kHidden) / kHeadDim;
-    half_t* const out = part == 0 ? p.q : part == 1 ? p.k : p.v;
+    // By value: between the members themselves the choice is one of addresses,
+    // which keeps the whole struct in scratch memory.
+    half_t* const q = p.q;
+    half_t* const k = p.k;
+    half_t* const v = p.v;
+    half_t* out = q;
+    if (part == 1) out = k;
+    if (part == 2) out = v;
     const size_t head_elems = (size_t)p.tpad * kHeadDim;
     const int rows16 = rope_table_rows(p.grid);
     // The tile's rows lie in images img0 .. img0 + BM / Tok + 1 (img0
@@ -278,7 +286,8 @@ __device__ __forceinline__ void qkv_epilogue(const QkvArgs& p, const Acc<T>& acc
 // half-fragment (a row-major head row would take 32 separate 32-byte writes
 // per store instead). Launched with rope_lds_bytes(grid) of dynamic LDS.
 template <class T, bool LN>
-__global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2) void qkv_rope_kernel(QkvArgs p) {
+__global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2) void qkv_rope_kernel(DHX_QKV_PARAMS) {
+    const QkvArgs p{h_, w_, bias_, cos_, sin_, q_, k_, v_, images_, grid_, tpad_, stats_, wsum_};
     static_assert(T::TN % kHeadDim == 0 && kHidden % T::BN == 0 && T::WGN == 1,
                   "whole heads per wave and tile, whole rows per wave");
         __shared__ __attribute__((aligned(16))) half_t wb0[T::WF_HALFS], wb1[T::WF_HALFS], wb2[T::WF_HALFS];
@@ -348,7 +357,8 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
 // load; here up to four 64-deep stages are in flight. At 201 rows 5.1 -> 4.7
 // us alone with warm caches, 2.3 us per launch less in the forward.
 template <class T, int NST, bool LN>
-__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void qkv_ring_kernel(QkvArgs p) {
+__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void qkv_ring_kernel(DHX_QKV_PARAMS) {
+    const QkvArgs p{h_, w_, bias_, cos_, sin_, q_, k_, v_, images_, grid_, tpad_, stats_, wsum_};
     static_assert(T::TN % kHeadDim == 0 && kHidden % T::BN == 0, "whole heads per wave and tile");
     DHX_RING_BUFS(T, NST);
     __shared__ __attribute__((aligned(16))) float bias[dma_copy_bytes(T::BN * 4) / 4], wsum[dma_copy_bytes(T::BN * 4) / 4];
@@ -466,7 +476,8 @@ __device__ __forceinline__ void resid_epilogue(const ResidArgs& p, const Acc<T>&
 // in fragment order (with STATS, also the LayerNorm row statistics of the
 // updated x); LDS holds only the weight stages and the column constants.
 template <class T, bool STATS, int KT = 0>
-__global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel(ResidArgs p) {
+__global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel(DHX_RESID_PARAMS) {
+    const ResidArgs p{a_, w_, bias_, ls_, x_, rows_, k_, stats_};
     static_assert(T::TN % 64 == 0 && T::TM == 32, "whole statistics slots, one 32-row block per wave");
     static_assert(T::BN <= T::THREADS, "one thread per column constant");
     constexpr int XF = T::TN / 16;  // x fragments per wave
@@ -517,7 +528,8 @@ __global__ __launch_bounds__(T::THREADS, T::BK == 128 ? 3 : 4) void resid_kernel
 // old x fragments, used only after every load has landed, are the only
 // register loads.
 template <class T, int NST, bool STATS, int KT>
-__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void resid_ring_kernel(ResidArgs p) {
+__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void resid_ring_kernel(DHX_RESID_PARAMS) {
+    const ResidArgs p{a_, w_, bias_, ls_, x_, rows_, k_, stats_};
     static_assert(T::BN <= T::THREADS, "one thread per column constant");
     DHX_RING_BUFS(T, NST);
     __shared__ __attribute__((aligned(16))) float raw_b[dma_copy_bytes(T::BN * 4) / 4], raw_l[dma_copy_bytes(T::BN * 4) / 4];
@@ -616,7 +628,8 @@ __device__ __forceinline__ void swiglu_mean(Acc<T>& acc, int i, const float* wsu
 // NS: N slices of the XCD tile split (xcd_tile_split); the launcher picks
 // it by the launch's size.
 template <class T, bool LN, int NS>
-__global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(SwigluArgs p) {
+__global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(DHX_SWIGLU_PARAMS) {
+    const SwigluArgs p{h_, w_, bias_, act_, rows_, stats_, wsum_};
     static_assert(T::TN % 64 == 0 && T::WGN == 1, "whole gate/up pairs, whole rows per wave");
     static_assert(T::BN <= T::THREADS, "one thread per column constant");
     static_assert(kHidden / T::BK > T::FN, "a K-loop step for every column block's LayerNorm mean term");
@@ -681,7 +694,8 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(
 // block b (of each 128 columns) before K step 64(b + 1), as in swiglu_kernel,
 // so a row's result is bitwise the same on either.
 template <class T, int NST, bool LN>
-__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void swiglu_ring_kernel(SwigluArgs p) {
+__global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void swiglu_ring_kernel(DHX_SWIGLU_PARAMS) {
+    const SwigluArgs p{h_, w_, bias_, act_, rows_, stats_, wsum_};
     static_assert(T::TN % 64 == 0, "whole gate/up pairs");
     static_assert(T::BN <= T::THREADS && T::BK <= 64, "one thread per column constant");
     DHX_RING_BUFS(T, NST);
@@ -741,7 +755,8 @@ struct SplitActFrags : ActFrags<T> {
 };
 
 template <class T, int KT = 0>
-__global__ __launch_bounds__(T::THREADS, 3) void splitk_kernel(SplitKArgs p) {
+__global__ __launch_bounds__(T::THREADS, 3) void splitk_kernel(DHX_SPLITK_PARAMS) {
+    const SplitKArgs p{a_, w_, partials_, rows_, k_, splits_};
     __shared__ __attribute__((aligned(16))) half_t wb0[T::WF_HALFS], wb1[T::WF_HALFS], wb2[T::WF_HALFS];
     constexpr int NT = kHidden / T::BN;
     const int MT = (p.rows + T::BM - 1) / T::BM;

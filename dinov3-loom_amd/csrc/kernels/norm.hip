@@ -22,7 +22,8 @@ constexpr int kLnKs = kKs / kWaves;     // blocks per wave in the LayerNorm
 // through LDS so that each wave writes 384-byte row runs.
 constexpr int kOutPitch = kLnKs * 16 + 4;  // floats per staged row of a wave
 
-__global__ __launch_bounds__(kThreads) void layernorm_kernel(LayerNormArgs p) {
+__global__ __launch_bounds__(kThreads) void layernorm_kernel(DHX_LAYERNORM_PARAMS) {
+    const LayerNormArgs p{x_, gamma_, beta_, out_, rows_, f32_out_};
     __shared__ float part[2][kWaves][32];
     __shared__ __attribute__((aligned(16))) float stage[kWaves][32 * kOutPitch];
     const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5, w = threadIdx.x >> 6;
@@ -93,7 +94,8 @@ __global__ __launch_bounds__(kThreads) void layernorm_kernel(LayerNormArgs p) {
 // STATS, the slot partials (mean, M2) of the updated f16 rows are written as
 // well (combined with the partner lane l ^ 32).
 template <bool STATS>
-__global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(ReduceArgs p) {
+__global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(DHX_REDUCE_PARAMS) {
+    const ReduceArgs p{partials_, bias_, ls_, x_, rows_, splits_, stats_};
     const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
     const int wid = blockIdx.x * kWaves + (threadIdx.x >> 6);
     const int mb = wid / kStatSlots, slot = wid % kStatSlots;
@@ -140,7 +142,8 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(ReduceArgs p) {
 
 // One thread per 16-byte piece of a padding row (8 per 64-channel row) of
 // each (tensor, image, head).
-__global__ __launch_bounds__(kThreads) void zero_pad_rows_kernel(PadRowsArgs p) {
+__global__ __launch_bounds__(kThreads) void zero_pad_rows_kernel(DHX_PAD_ROWS_PARAMS) {
+    const PadRowsArgs p{q_, k_, v_, images_, tokens_, tpad_};
     const int pad = p.tpad - p.tokens;
     const size_t per_tensor = (size_t)p.images * kHeads * pad * 8;
     const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
@@ -158,21 +161,18 @@ __global__ __launch_bounds__(kThreads) void zero_pad_rows_kernel(PadRowsArgs p) 
 hipError_t launch_zero_pad_rows(const PadRowsArgs& a, hipStream_t s) {
     const size_t n = 3ull * a.images * kHeads * (a.tpad - a.tokens) * 8;
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(zero_pad_rows_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, a);
-    return hipGetLastError();
+    return start(zero_pad_rows_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, a);
 }
 
 hipError_t launch_layernorm(const LayerNormArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL(layernorm_kernel, dim3((a.rows + 31) / 32), dim3(kThreads), 0, s, a);
-    return hipGetLastError();
+    return start(layernorm_kernel, dim3((a.rows + 31) / 32), dim3(kThreads), 0, s, a);
 }
 
 hipError_t launch_splitk_reduce(const ReduceArgs& a, hipStream_t s) {
     const int waves = (a.rows + 31) / 32 * kStatSlots;
     const int blocks = (waves + kWaves - 1) / kWaves;
-    if (a.stats) hipLaunchKernelGGL(splitk_reduce_kernel<true>, dim3(blocks), dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL(splitk_reduce_kernel<false>, dim3(blocks), dim3(kThreads), 0, s, a);
-    return hipGetLastError();
+    return a.stats ? start(splitk_reduce_kernel<true>, dim3(blocks), dim3(kThreads), 0, s, a)
+                   : start(splitk_reduce_kernel<false>, dim3(blocks), dim3(kThreads), 0, s, a);
 }
 
 }  // namespace dhx
