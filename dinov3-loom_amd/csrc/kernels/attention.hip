@@ -3,10 +3,9 @@
 //
 // Three kernels share one step (attend32), each wave owning 32 queries of one
 // (image, head) and taking 32 keys a step: attention_kernel (four waves walk
-// all keys), attention_resident_kernel (the same with every key block in
-// flight at once, for short sequences in small launches) and
-// attention_split_kernel (two key halves, for long sequences); the launcher
-// says which runs when. Keys stream through LDS in blocks of 32 or 64 (K and
+// all keys), attention_parallel_kernel (a wave per key block, for short
+// sequences in small launches) and attention_split_kernel (two key halves, for
+// long sequences); the launcher says which runs when. Keys stream through LDS in blocks of 32 or 64 (K and
 // V both as [key][ch]). q, k and v come per (image, head) as [tpad][64]
 // matrices in fragment order (a wave's Q fragments are then 1 KB contiguous
 // loads). The blocks move from global memory straight into LDS with DMA loads
@@ -66,15 +65,6 @@ __device__ __forceinline__ void vm_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// Calls f(integral_constant<int, I>) for I = 0 .. N-1.
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void for_constants(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        for_constants<N, I + 1>(f);
-    }
-}
-
 // The running softmax state of one lane's query (lane l holds query l % 32
 // and half of each 32-key sub-block's scores; see the top of this file).
 struct QueryState {
@@ -127,119 +117,140 @@ struct LaneOffsetsXor {
     __device__ __forceinline__ int v(int ct, int r) const { return (v_ ^ (ct << 5) ^ (r << 4)) + r * 8 * kHeadDim; }
 };
 
-// One sub-block of 32 keys (rows row0 .. row0+31 of the swizzled K and V
-// blocks in LDS, keys key0 .. key0+31 of the sequence of T):
-// S^T = K Q^T, masked past T, lazy running max, P = 2^(s log2e - m log2e),
+// The pieces of one step over a 32-key block (keys key0 .. key0+31 of the
+// sequence of T). Scores: s[r] is that of key key0 + 8(r/4) + 4*hi + r%4 for
+// query l32 (S^T = K Q^T), -inf past T.
+template <class Offsets>
+__device__ __forceinline__ float16_t scores32(const half_t* sK, const half8_t (&qf)[4], const Offsets& at) {
+    float16_t s = {};
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) s = mfma32x32x16(*(const half8_t*)(sK + at.k(kk)), qf[kk], s);
+    return s;
+}
+
+__device__ __forceinline__ void mask32(float16_t& s, int key0, int T, int hi) {
+    if (key0 + 32 > T) {  // the last, partial block of keys (uniform)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            if (key0 + 8 * (r >> 2) + 4 * hi + (r & 3) >= T) s[r] = -__builtin_inff();
+    }
+}
+
+// V^T operand of channels ct*32 + l32 and keys key0 + 16ks + (j < 4 ? 4hi + j
+// : 8 + 4hi + j - 4).
+template <class Offsets>
+__device__ __forceinline__ half8_t v_frag(const half_t* sV, int ct, int ks, const Offsets& at) {
+    const half4_t a0 = lds_read_tr16(sV + ks * 16 * kHeadDim + at.v(ct, 0));
+    const half4_t a1 = lds_read_tr16(sV + ks * 16 * kHeadDim + at.v(ct, 1));
+    return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// p = 2^(s log2e - m log2e); returns the sum over the lane pair.
+__device__ __forceinline__ float weights32(const float16_t& s, float m, float (&p)[16]) {
+    const float mb = m * kLog2e;
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        p[r] = fast_exp2(fmaf(s[r], kLog2e, -mb));
+        sum += p[r];
+    }
+    return half_pair_sum(sum);
+}
+
+__device__ __forceinline__ float block_max32(const float16_t& s) {
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    return half_pair_max(mx);  // every block holds a valid key of each pair
+}
+
+// P^T as the b operand: k-slice element j of this lane is the key of v_frag's
+// element j.
+__device__ __forceinline__ half8_t p_frag(const float (&p)[16], int ks) {
+    half8_t b;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) b[e] = (half_t)p[8 * ks + e];
+    return b;
+}
+
+// One step over a 32-key block (rows row0 .. row0+31 of the swizzled K and V
+// blocks in LDS): scores, lazy running max, weights P = 2^(s log2e - m log2e),
 // O^T += V^T P^T with P in f16 and the denominator in f32. FIRST: the first
-// sub-block of a walk (O and l still zero), whose weights against the
-// initial max of -1e30 would all overflow: its block max becomes the
-// running max directly, with one pass of exponentials instead of two (the
-// same values and rounding as the rescale path).
+// block of a walk (O and l still zero), whose weights against the initial max
+// of -1e30 would all overflow: its block max becomes the running max directly,
+// with one pass of exponentials instead of two (the same values and rounding
+// as the rescale path).
 template <bool FIRST = false, class Offsets>
 __device__ __forceinline__ void attend32(QueryState& st, const half_t* sK, const half_t* sV, int row0, int key0,
                                          int T, int lane, Offsets& at) {
     at.step();
-    const int hi = lane >> 5;
-    const float neg_inf = -__builtin_inff();
-    float16_t s = {};
     sK += row0 * kHeadDim;
     sV += row0 * kHeadDim;
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) s = mfma32x32x16(*(const half8_t*)(sK + at.k(kk)), st.qf[kk], s);
+    float16_t s = scores32(sK, st.qf, at);
     // The V^T operands do not depend on the softmax: read them now so their
-    // LDS latency hides under the exponentials. va[ct][ks] holds channel
-    // ct*32 + l32 of keys key0 + 16ks + (j < 4 ? 4hi + j : 8 + 4hi + j - 4).
+    // LDS latency hides under the exponentials.
     half8_t va[2][2];
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const half4_t a0 = lds_read_tr16(sV + ks * 16 * kHeadDim + at.v(ct, 0));
-            const half4_t a1 = lds_read_tr16(sV + ks * 16 * kHeadDim + at.v(ct, 1));
-            va[ct][ks] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
-    // s[r] is the score of key key0 + 8(r/4) + 4*hi + r%4 for query l32.
-    if (key0 + 32 > T) {  // the last, partial block of keys (uniform)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            if (key0 + 8 * (r >> 2) + 4 * hi + (r & 3) >= T) s[r] = neg_inf;
-    }
-    // Weights against the running max; after the first sub-block (which
-    // takes its own max), the block max is needed only when some lane's
-    // weights sum past e^8 (a weight may then exceed it): blocks whose
-    // scores grew by more than 8. Those lanes move their max to the
-    // block's, rescale O and l, and recompute; every weight is then at most
-    // its sum, at most e^8, well inside f16.
-    float p[16];
-    auto weights = [&](float m) {  // p = 2^(s log2e - m log2e); the pair's sum
-        const float mb = m * kLog2e;
-        float sum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            p[r] = fast_exp2(fmaf(s[r], kLog2e, -mb));
-            sum += p[r];
-        }
-        return half_pair_sum(sum);
-    };
-    auto block_max = [&] {
-        float mx = s[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-        return half_pair_max(mx);  // every sub-block holds a valid key of each pair
-    };
-    float sum;
+        for (int ks = 0; ks < 2; ++ks) va[ct][ks] = v_frag(sV, ct, ks, at);
+    mask32(s, key0, T, lane >> 5);
+    // Weights against the running max; after the first block (which takes its
+    // own max), the block max is needed only when some lane's weights sum past
+    // e^8 (a weight may then exceed it): blocks whose scores grew by more than
+    // 8. Those lanes move their max to the block's, rescale O and l, and
+    // recompute; every weight is then at most its sum, at most e^8, well
+    // inside f16.
+    float p[16], sum;
     if constexpr (FIRST) {
-        st.m_run = block_max();
-        sum = weights(st.m_run);
+        st.m_run = block_max32(s);
+        sum = weights32(s, st.m_run, p);
     } else {
-        sum = weights(st.m_run);
+        sum = weights32(s, st.m_run, p);
         const bool grow = !(sum <= kLazySum);
         if (__any(grow)) {  // uniform across the wave
-            const float m_new = grow ? fmaxf(block_max(), st.m_run) : st.m_run;
+            const float m_new = grow ? fmaxf(block_max32(s), st.m_run) : st.m_run;
             const float alpha = fast_exp2((st.m_run - m_new) * kLog2e);
             st.l_run *= alpha;
             st.o[0] *= alpha;
             st.o[1] *= alpha;
             st.m_run = m_new;
-            sum = weights(m_new);
+            sum = weights32(s, m_new, p);
         }
     }
     st.l_run += sum;
-    // P^T as the b operand: k-slice element j of this lane is key
-    // key0 + 16ks + (j < 4 ? 4hi + j : 8 + 4hi + j - 4), as in va.
-    half8_t pb[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) pb[ks][e] = (half_t)p[8 * ks + e];
+    const half8_t pb[2] = {p_frag(p, 0), p_frag(p, 1)};
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) st.o[ct] = mfma32x32x16(va[ct][ks], pb[ks], st.o[ct]);
 }
 
-// Output of one lane's query: O / l in f16 into out (fragment order): each
-// 16-channel half of a 32-channel block becomes one 8-channel piece per lane
-// after frag_swap. row0: the first query row of the wave (wave-uniform); the
-// wave's 32 rows lie in its 32-row block and the next, which the
+// Output of one lane's query, channel half ct: O / l in f16 into out (fragment
+// order): each 16-channel half of the block becomes one 8-channel piece per
+// lane after frag_swap. row0: the first query row of the wave (wave-uniform);
+// the wave's 32 rows lie in its 32-row block and the next, which the
 // write-through descriptor covers.
-__device__ __forceinline__ void store_query(const QueryState& st, half_t* out, int row0, int row, int head, int hi) {
+__device__ __forceinline__ void store_half(const float16_t& a, float inv, half_t* out, int row0, int row, int head,
+                                           int ct, int hi) {
     const size_t base = (size_t)(row0 / 32) * (kHidden / 16) * 512;
     const WtOut o(out + base, 2 * (kHidden / 16) * 1024);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+        const half4_t g0 = {(half_t)(a[8 * kk] * inv), (half_t)(a[8 * kk + 1] * inv),
+                            (half_t)(a[8 * kk + 2] * inv), (half_t)(a[8 * kk + 3] * inv)};
+        const half4_t g1 = {(half_t)(a[8 * kk + 4] * inv), (half_t)(a[8 * kk + 5] * inv),
+                            (half_t)(a[8 * kk + 6] * inv), (half_t)(a[8 * kk + 7] * inv)};
+        const half8_t piece = frag_swap(g0, g1);
+        const int c = head * kHeadDim + ct * 32 + kk * 16 + hi * 8;
+        o.store((uint32_t)(frag_piece(row, c, kHidden) - base) * 2, piece);
+    }
+}
+
+__device__ __forceinline__ void store_query(const QueryState& st, half_t* out, int row0, int row, int head, int hi) {
     const float inv = 1.0f / st.l_run;
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const float16_t& a = st.o[ct];
-            const half4_t g0 = {(half_t)(a[8 * kk] * inv), (half_t)(a[8 * kk + 1] * inv),
-                                (half_t)(a[8 * kk + 2] * inv), (half_t)(a[8 * kk + 3] * inv)};
-            const half4_t g1 = {(half_t)(a[8 * kk + 4] * inv), (half_t)(a[8 * kk + 5] * inv),
-                                (half_t)(a[8 * kk + 6] * inv), (half_t)(a[8 * kk + 7] * inv)};
-            const half8_t piece = frag_swap(g0, g1);
-            const int c = head * kHeadDim + ct * 32 + kk * 16 + hi * 8;
-            o.store((uint32_t)(frag_piece(row, c, kHidden) - base) * 2, piece);
-        }
+    for (int ct = 0; ct < 2; ++ct) store_half(st.o[ct], inv, out, row0, row, head, ct, hi);
 }
 
 // NKB > 0: the number of key blocks of KB = 32 keys, known at compile time
@@ -406,78 +417,116 @@ __global__ __launch_bounds__(kThreads, 3) void attention_kernel(DHX_ATTENTION_PA
     if (qrow < T) store_query(st, p.out, img * T + qb * QB + wave * 32, img * T + qrow, head, hi);
 }
 
-// Short sequences in launches of at most one workgroup per CU: all N = ceil(T
-// / 32) key blocks are in flight from the start, each with LDS of its own
-// (8 KB per block), so a workgroup waits for one load latency instead of one
-// per block or two: one block 3.6 -> 3.0 us per launch, four 4.5 -> 3.8, five
-// 4.8 -> 4.2, six 5.2 -> 4.6 (HIP events, alone). At seven blocks (201 tokens)
-// the softmax chain of a wave, about 0.4 us per block, covers the loads in
-// attention_kernel already (5.34 -> 5.25 us, the forward unchanged). The Q
-// fragments come through LDS as well (4 KB per wave): with DMA loads only,
-// every wait is an exact count. The steps are those of attention_kernel, so a
-// query's result is bitwise the same.
-constexpr int kMaxResident = 6;
+// Short sequences in small launches: a workgroup holds 32 queries, and wave j
+// of its N = ceil(T / 32) takes key block j. In attention_kernel a wave walks
+// the blocks one after another, and a small launch waits for that chain of N
+// softmax steps (about 0.4 us each) on a few SIMDs. Here the blocks' scores,
+// weights and weight sums are taken side by side, against the first block's
+// max: where no later block's weights against it sum past e^8, that is the
+// running max attention_kernel keeps too. Then two waves, one per 32
+// channels, run the PV products over the blocks in order, and the sums are
+// added in order, so a query's result is bitwise that of attention_kernel.
+// Where some block's weights do sum past e^8, the first wave walks the blocks
+// as attention_kernel would. All loads are DMA, with exact waits. Alone: 201
+// tokens 5.1 -> 4.2 us to 6 images, 69 tokens 4.25 -> 3.0, 261 tokens 6.5 ->
+// 5.2, 405 tokens 8.0 -> 6.4; what is left is the launch, the loads, one
+// softmax step and the 2 N MFMAs of a PV chain.
+constexpr int kMaxParallel = 15;
 
-// Halfs of a ring's or a resident set's i-th 32-key block out of N (a
-// placeholder past the last).
 template <int N>
-struct BlockLds {
-    template <int I>
-    static constexpr int at = I < N ? 32 * kHeadDim : 8;
+struct ParallelLds {
+    static constexpr int KV = N * 32 * kHeadDim;  // halfs of K (or V)
+    static constexpr int P = N * 2 * 512;         // halfs of P^T fragments
+    static constexpr int SUMS = N * 32;
 };
 
 template <int N>
-__device__ __forceinline__ void resident_walk(QueryState& st, half_t* const (&kbuf)[kMaxResident],
-                                              half_t* const (&vbuf)[kMaxResident], half_t* sq,
-                                              const __amdgpu_buffer_rsrc_t& rq, const __amdgpu_buffer_rsrc_t& rk,
-                                              const __amdgpu_buffer_rsrc_t& rv, int q0, int T, int wave, int lane) {
+__device__ __forceinline__ void parallel_blocks(const AttentionArgs& p, half_t* sk, half_t* sv, half_t* sq, half_t* sp,
+                                                float* smax, float* sums, int* grew, int qb, int head, int img) {
+    constexpr int BLK = 32 * kHeadDim;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hi = lane >> 5, T = p.tokens, q0 = qb * 32;
+    const HeadSrc src(p, img, head);
     auto lds = [](half_t* a) { return (__attribute__((address_space(3))) void*)a; };
-    // The wave's 32 query rows (rows past T are tpad's padding: finite, and
-    // never stored), then its 8 rows of every key block.
+    // Q fragment kk by wave kk % N (rows past T are tpad's padding: finite, and
+    // never stored), then the wave's own K block and V block.
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, lds(sq + kk * 512), 16, lane * 16, (q0 / 32 * 4 + kk) * 1024, 0, 0);
-    const int row = wave * 8, voff = dma_lane_offset(lane, row);
+        if (kk % N == wave)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(src.q, lds(sq + kk * 512), 16, lane * 16, (qb * 4 + kk) * 1024, 0, 0);
+    half_t* const k_own = sk + wave * BLK;
+    half_t* const v_own = sv + wave * BLK;
+    const int even = dma_lane_offset(lane, 0), odd = dma_lane_offset(lane, 8);
 #pragma unroll
-    for (int kb = 0; kb < N; ++kb) {
-        const int soff = dma_row_offset(kb * 32 + row);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, lds(kbuf[kb] + row * kHeadDim), 16, voff, soff, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, lds(vbuf[kb] + row * kHeadDim), 16, voff, soff, 0, 0);
-    }
-    st.o[0] = st.o[1] = float16_t{};
+    for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src.k, lds(k_own + 8 * i * kHeadDim), 16, i & 1 ? odd : even,
+                                                 dma_row_offset(wave * 32 + 8 * i), 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src.v, lds(v_own + 8 * i * kHeadDim), 16, i & 1 ? odd : even,
+                                                 dma_row_offset(wave * 32 + 8 * i), 0, 0);
+    if (tid == 0) *grew = 0;
     LaneOffsets at(lane);
-    const bool active = q0 < T;  // waves whose queries all lie past T only move K and V
-    for_constants<N>([&](auto KB) {
-        constexpr int kb = decltype(KB)::value;
-        if constexpr (kb == 0) {
-            vm_barrier<2 * N - 1>();  // Q has landed (and the first K block)
+    QueryState st;
+    vm_barrier<4>();  // Q and K have landed; V may be outstanding
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) st.qf[kk] = *(const half8_t*)(sq + kk * 512 + lane * 8) * (half_t)0.125f;
+    for (int kk = 0; kk < 4; ++kk) st.qf[kk] = *(const half8_t*)(sq + kk * 512 + lane * 8) * (half_t)0.125f;
+    float16_t s = scores32(k_own, st.qf, at);
+    mask32(s, wave * 32, T, hi);
+    if (wave == 0) smax[l32] = block_max32(s);  // both lanes of a pair hold the pair's
+    vm_barrier<0>();
+    float w[16];
+    const float sum = weights32(s, smax[l32], w);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) *(half8_t*)(sp + (wave * 2 + ks) * 512 + lane * 8) = p_frag(w, ks);
+    sums[wave * 32 + l32] = sum;
+    if (wave > 0 && __any(!(sum <= kLazySum))) *grew = 1;
+    vm_barrier<0>();
+    const int row0 = img * T + q0, row = row0 + l32;
+    if (*grew) {  // uniform across the workgroup
+        if (wave > 0) return;
+        st.o[0] = st.o[1] = float16_t{};
+        attend32<true>(st, sk, sv, 0, 0, T, lane, at);
+        for (int kb = 1; kb < N; ++kb) attend32(st, sk + kb * BLK, sv + kb * BLK, 0, kb * 32, T, lane, at);
+        if (q0 + l32 < T) store_query(st, p.out, row0, row, head, hi);
+        return;
+    }
+    float l = sums[l32];
+#pragma unroll
+    for (int kb = 1; kb < N; ++kb) l += sums[kb * 32 + l32];
+    const float inv = 1.0f / l;
+    if (wave > 1) return;
+#pragma unroll
+    for (int c = 0; c < (N == 1 ? 2 : 1); ++c) {
+        const int ct = N == 1 ? c : wave;
+        // Channel half 1 sits 4 chunks from half 0 (LaneOffsets, one exclusive or).
+        const half_t* const v0 = sv + (at.v(0, 0) ^ (ct << 5));
+        const half_t* const v1 = sv + (at.v(0, 1) ^ (ct << 5));
+        float16_t o = {};
+#pragma unroll
+        for (int b = 0; b < 2 * N; ++b) {  // 16-key slices: block b / 2
+            const half4_t a0 = lds_read_tr16(v0 + b * 16 * kHeadDim), a1 = lds_read_tr16(v1 + b * 16 * kHeadDim);
+            o = mfma32x32x16(__builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7),
+                             *(const half8_t*)(sp + b * 512 + lane * 8), o);
         }
-        vm_barrier<2 * (N - 1 - kb)>();  // only later blocks may be outstanding
-        if (active) attend32<kb == 0>(st, kbuf[kb], vbuf[kb], 0, kb * 32, T, lane, at);
-    });
+        if (q0 + l32 < T) store_half(o, inv, p.out, row0, row, head, ct, hi);
+    }
 }
 
+// As many waves per SIMD as two workgroups per CU have (one from eight blocks
+// on, by its LDS).
 template <int N>
-__global__ __launch_bounds__(kThreads, 2) void attention_resident_kernel(DHX_ATTENTION_PARAMS) {
+__global__ __launch_bounds__(N * kWave, N > 7 ? (N + 3) / 4 : N > 3 ? (N + 1) / 2 : 2) void attention_parallel_kernel(
+    DHX_ATTENTION_PARAMS) {
     const AttentionArgs p{q_, k_, v_, out_, images_, tokens_, tpad_};
-    using L = BlockLds<N>;
-    __shared__ __attribute__((aligned(16))) half_t k0[L::template at<0>], k1[L::template at<1>], k2[L::template at<2>], k3[L::template at<3>], k4[L::template at<4>], k5[L::template at<5>];
-    __shared__ __attribute__((aligned(16))) half_t v0[L::template at<0>], v1[L::template at<1>], v2[L::template at<2>], v3[L::template at<3>], v4[L::template at<4>], v5[L::template at<5>];
-    __shared__ __attribute__((aligned(16))) half_t sq[4 * 4 * 512];  // four fragments per wave
-    const int nqb = (p.tokens + QB - 1) / QB, total = nqb * kHeads * p.images;
+    using L = ParallelLds<N>;
+    __shared__ __attribute__((aligned(16))) half_t sk[L::KV], sv[L::KV], sq[4 * 512], sp[L::P];
+    __shared__ float smax[32], sums[L::SUMS];
+    __shared__ int grew;
+    const int nqb = (p.tokens + 31) / 32, total = nqb * kHeads * p.images;
     const int per = (total + 7) >> 3, g = blockIdx.x, t = (g & 7) * per + (g >> 3);
     if ((g >> 3) >= per || t >= total) return;  // uniform per workgroup
-    const int qb = t % nqb, head = (t / nqb) % kHeads, img = t / (nqb * kHeads);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int q0 = qb * QB + wave * 32, q = q0 + (lane & 31);
-    const HeadSrc src(p, img, head);
-    half_t* const kbuf[kMaxResident] = {k0, k1, k2, k3, k4, k5};
-    half_t* const vbuf[kMaxResident] = {v0, v1, v2, v3, v4, v5};
-    QueryState st;
-    resident_walk<N>(st, kbuf, vbuf, sq + wave * 2048, src.q, src.k, src.v, q0, p.tokens, wave, lane);
-    if (q < p.tokens) store_query(st, p.out, img * p.tokens + q0, img * p.tokens + q, head, lane >> 5);
+    parallel_blocks<N>(p, sk, sv, sq, sp, smax, sums, &grew, t % nqb, (t / nqb) % kHeads, t / (nqb * kHeads));
 }
 
 // Long sequences: workgroups of 2 QW waves hold 32 QW queries as QW query
@@ -652,10 +701,10 @@ constexpr int kSplitBlocks = 16;  // blocks of 32 keys, from 481 tokens on
 constexpr int kRound = 256;       // workgroups of one per CU
 
 template <int N>
-hipError_t launch_resident(const AttentionArgs& a, int nkb, dim3 grid, hipStream_t s) {
+hipError_t launch_parallel(const AttentionArgs& a, int nkb, int groups, hipStream_t s) {
     if constexpr (N > 1)
-        if (nkb < N) return launch_resident<N - 1>(a, nkb, grid, s);
-    return start(attention_resident_kernel<N>, grid, dim3(kThreads), 0, s, a);
+        if (nkb < N) return launch_parallel<N - 1>(a, nkb, groups, s);
+    return start(attention_parallel_kernel<N>, dim3((groups + 7) & ~7), dim3(N * kWave), 0, s, a);
 }
 
 template <int NH, int QW>
@@ -665,24 +714,28 @@ hipError_t launch_split(const AttentionArgs& a, int groups, hipStream_t s) {
 
 }  // namespace
 
-// 224x224 (201 tokens): seven blocks of 32 keys, unrolled. Fewer blocks in
-// launches of at most one workgroup per CU: all resident. From 481 tokens on
-// two key halves, on workgroups of 64 queries where one round of them covers
-// the launch, which then runs on twice the CUs with one wave per SIMD (whole
-// forward, 128 -> 64 queries: 384x384 batch 3 439 -> 421 us, 512x512 batch 1
-// 455 -> 424, 720x720 batch 1 620 -> 569; attention_kernel with its run-time
-// count before: 443, -, 666), else of 128 (1024x1024 batch 2 1852 -> 1800;
-// equal to attention_kernel from 581 tokens on, 5 % slower at 405). 512x512
-// (17 blocks per half) in more than one round takes the unrolled walk (batch 8
-// 975 -> 964 us); in one round its 80 KB of code cost more to fetch than they
-// save (batch 1 449 against 424, batch 4 636 against 629). Otherwise blocks of
-// 64 keys with a run-time count.
+// To 480 tokens, where one round of 32-query workgroups covers the launch, one
+// wave per key block (whole forward, against the walks below: 224x224 batch 1
+// 304 -> 294 us, batch 6 332 -> 322, 128x128 batch 4 302 -> 286, 256x256 batch
+// 4 351 -> 334, 320x320 batch 3 368 -> 349; in two rounds 224x224 batch 8 351
+// -> 361). From 481 tokens on two key halves, on workgroups of 64 queries
+// where one round of them covers the launch, which then runs on twice the CUs
+// with one wave per SIMD (128 -> 64 queries: 384x384 batch 3 439 -> 421 us,
+// 512x512 batch 1 455 -> 424, 720x720 batch 1 620 -> 569; attention_kernel with
+// its run-time count before: 443, -, 666), else of 128 (1024x1024 batch 2 1852
+// -> 1800; equal to attention_kernel from 581 tokens on, 5 % slower at 405).
+// 512x512 (17 blocks per half) in more than one round takes the unrolled walk
+// (batch 8 975 -> 964 us); in one round its 80 KB of code cost more to fetch
+// than they save (batch 1 449 against 424, batch 4 636 against 629). 201
+// tokens: seven blocks of 32 keys, unrolled. Otherwise blocks of 64 keys with
+// a run-time count.
 hipError_t launch_attention(const AttentionArgs& a, hipStream_t s) {
     const int nqb = (a.tokens + QB - 1) / QB, total = nqb * kHeads * a.images;
     const int total64 = (a.tokens + 63) / 64 * kHeads * a.images;
     const dim3 grid((total + 7) & ~7), block(kThreads);
     const int nkb = (a.tokens + 31) / 32;
-    if (nkb <= kMaxResident && total <= kRound) return launch_resident<kMaxResident>(a, nkb, grid, s);
+    const int total32 = nkb * kHeads * a.images;
+    if (nkb <= kMaxParallel && total32 <= kRound) return launch_parallel<kMaxParallel>(a, nkb, total32, s);
     if (nkb >= kSplitBlocks) {
         if (total64 <= kRound) return launch_split<0, 2>(a, total64, s);
         if ((nkb + 1) / 2 == 17 && total > kRound) return launch_split<17, 4>(a, total, s);

@@ -1,8 +1,8 @@
 """Every attention kernel a sequence can run on gives an image the same bits:
-launches on both sides of each rule's edge (one workgroup per CU for the
-resident and the 64-query kernels, one round for the unrolled walk) against
-one larger launch of the same images, and the sequences around the edge of the
-two-halves walk against the float64 oracle."""
+launches on both sides of each rule's edge (one round of workgroups for the
+wave-per-block and the 64-query kernels, more than one for the unrolled walk)
+against one larger launch of the same images, and the sequences around the
+edge of the two-halves walk against the float64 oracle."""
 import numpy as np
 import pytest
 
@@ -28,18 +28,24 @@ def inputs(grid, images, scale=2.0):
     return [f16(rng.normal(size=(rows, 384)) * s) for s in (scale, 1.0, 1.0)]
 
 
-# (grid, images of the large launch, images of the others): 1, 3, 5 and 6 key
-# blocks (resident up to 256 workgroups), 16 and 19 blocks (64-query
-# workgroups up to 256 of them), 1029 tokens (64 queries to 2 images, 128 from
-# 3, the unrolled walk from 5), 2030 tokens.
-ROUTES = [(4, 50, (1, 42, 43)), (8, 50, (1, 42, 43)), (12, 24, (1, 21, 22)), (13, 24, (1, 21, 22)),
-          (22, 8, (1, 5, 6)), (24, 8, (1, 4, 5)), (32, 6, (1, 2, 3, 4, 5)), (45, 3, (1, 2))]
+# (grid, images of the large launch, images of the others): 1, 3, 5, 7, 8, 9
+# and 14 key blocks (a wave per block up to 256 workgroups of 32 queries), 16
+# and 19 blocks (64-query workgroups up to 256 of them), 1029 tokens (64
+# queries to 2 images, 128 from 3, the unrolled walk from 5), 2030 tokens.
+ROUTES = [(4, 50, (1, 42, 43)), (8, 20, (1, 14, 15)), (12, 12, (1, 8, 9)), (14, 10, (1, 6, 7)), (15, 8, (1, 5, 6)),
+          (16, 8, (1, 4, 5)), (21, 6, (1, 3, 4)), (22, 8, (1, 5, 6)), (24, 8, (1, 4, 5)), (32, 6, (1, 2, 3, 4, 5)),
+          (45, 3, (1, 2))]
 
 
+# ramp: the scores grow along the keys, so the running max has to move.
+@pytest.mark.parametrize("ramp", [False, True])
 @pytest.mark.parametrize("grid,most,counts", ROUTES)
-def test_images_do_not_depend_on_the_launch(eng, grid, most, counts):  # noqa: F811
-    mats = inputs(grid, most)
+def test_images_do_not_depend_on_the_launch(eng, grid, most, counts, ramp):  # noqa: F811
+    q, k, v = inputs(grid, most)
     T = grid * grid + 5
+    if ramp:
+        k = f16(k * np.tile(np.linspace(0.1, 8.0, T), most)[:, None])
+    mats = [q, k, v]
     want = launch(eng, mats, most, grid)
     assert np.all(np.isfinite(want))
     for images in counts:
