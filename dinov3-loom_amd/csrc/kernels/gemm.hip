@@ -46,6 +46,7 @@ using SplitTile = Tile<128, 128, 4, 1>;
 
 // Tiles of the ring kernels, two to eight waves of 32x32 or 32x64.
 using ResidRing32 = Tile<32, 64, 1, 2, 128>;
+using ResidRing32K = Tile<32, 64, 1, 2, 64>;
 using ResidRing64 = Tile<64, 64, 2, 2, 64>;
 using ResidRing128 = Tile<128, 64, 4, 2, 64>;
 using ResidRing128W = Tile<128, 128, 4, 2, 64>;
@@ -95,7 +96,7 @@ static hipError_t launch_qkv_ring(const QkvArgs& a, hipStream_t s) {
 // 519 / 487, 4020 rows 513 / 645 / 583 / 559.
 hipError_t launch_qkv_rope(const QkvArgs& a, hipStream_t s) {
     const int rows = a.images * (a.grid * a.grid + kPrefix);
-    if (rows <= kRound / 18 * 64) return launch_qkv_ring<QkvRing64, 5>(a, s);
+    if (rows <= kRound / 18 * 64) return launch_qkv_ring<QkvRing64, 4>(a, s);
     if (rows <= kRound / 9 * 64) return launch_qkv_ring<QkvRing64W, 4>(a, s);
     if (rows <= kRound / 9 * 128) return launch_qkv_ring<QkvRing128, 3>(a, s);
     return rows < kQkvSmallRows ? launch_qkv_tiles<QkvTileS>(a, s) : launch_qkv_tiles<QkvTile>(a, s);
@@ -112,10 +113,13 @@ hipError_t launch_resid(const ResidArgs& a, hipStream_t s) {
     // Launches that one round of workgroups covers, one per CU, take the
     // smallest ring tile that does (N = 384 is six 64-column tiles): a smaller
     // one needs a second round, a larger one leaves CUs idle. Whole forward
-    // (one chain, graph replay): 32x64 for the o-projection at 201 rows 412 ->
-    // 403 us, 64x64 406; 64x64 for the down projection at 201 / 1005 / 2412
-    // rows 412 -> 376, 404 -> 368, 488 -> 455 us (32x64: 375, 367, 517), at
-    // 3216 rows 528 -> 551; 128x64 there 528 -> 517 and at 4020 rows 539 -> 527.
+    // (one chain, graph replay), against resid_kernel: o-projection 32x64 at
+    // 201 rows 412 -> 403 us (64x64 406); down projection 64x64 at 201 / 1005
+    // / 2412 rows 412 -> 376, 404 -> 368, 488 -> 455, at 3216 rows 528 -> 551;
+    // 128x64 there 528 -> 517 and at 4020 rows 539 -> 527. To 1344 rows the
+    // down projection's 32x64 tile with five 64-deep stages in flight takes
+    // 8.5 us off each of these (201 rows 295.3 -> 286.8, 1005 rows 315.6 ->
+    // 308.5; three or four 128-deep stages 294, 293, 1608 rows 355 -> 377).
     // Beside another image group's kernels (a.shared) the 128x64 ring, which
     // takes a CU's LDS whole, loses to the tiles below (705 -> 742 us at 2 x
     // 3216 rows).
@@ -131,7 +135,8 @@ hipError_t launch_resid(const ResidArgs& a, hipStream_t s) {
     if (a.k == kHidden && round == 32) return launch_resid_ring<ResidRing32, 4, kHidden>(a, s);
     if (a.k == kHidden && round == 64) return launch_resid_ring<ResidRing64, 5, kHidden>(a, s);
     if (a.k == kHidden && round == 128) return launch_resid_ring<ResidRing128, 4, kHidden>(a, s);
-    if (a.k == kFF && (round == 32 || round == 64)) return launch_resid_ring<ResidRing64, 5, kFF>(a, s);
+    if (a.k == kFF && round == 32) return launch_resid_ring<ResidRing32K, 6, kFF>(a, s);
+    if (a.k == kFF && round == 64) return launch_resid_ring<ResidRing64, 5, kFF>(a, s);
     if (a.k == kFF && round == 128) return launch_resid_ring<ResidRing128, 4, kFF>(a, s);
     if (a.k == kFF && round == 256) return launch_resid_ring<ResidRing128W, 4, kFF>(a, s);
     // The K loop walks its stages six at a time (gemm_main_dma).
