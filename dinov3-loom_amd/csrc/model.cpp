@@ -36,6 +36,15 @@ constexpr uint64_t kHiddenU = 384;
 constexpr uint32_t kSplits = 4;
 // Smallest image group worth its own branch of the plan.
 constexpr uint64_t kMinBranchImages = 4;
+// Batch rows (images * tokens) from which two groups are the default. Two
+// chains of half the rows fill each other's partial rounds of workgroups; but
+// below this the tiles chosen by size fit a whole launch in about one round,
+// and the second chain only takes compute units from the first. Replays of
+// one group | two, us: 224x224 8 images (1608 rows) 354 | 499, 16 (3216)
+// 459 | 497, 20 (4020) 483 | 545, 24 (4824) 564 | 559, 28 (5628) 675 | 619,
+// 64 (12864) 1167 | 1092; 384x384 8 images (4648 rows) 611 | 687, 10 (5810)
+// 783 | 755; 64x64 64 images (1344 rows) 341 | 442.
+constexpr uint64_t kTwoGroupRows = 4800;
 
 // hub.rs:7-11
 constexpr char kRepoOwner[] = "facebook";
@@ -318,19 +327,18 @@ public:
     }
 
     // lib.rs:149-263 (prepare): one launch plan per batch size, recorded as
-    // one graph. The batch is cut into `branches_` groups of images (for
-    // b >= 2 * kMinBranchImages) that run as independent chains, each over
-    // its own slice of every buffer: the kernels of one group fill the last,
-    // partial wave of workgroups of the other's. A row's arithmetic does not
-    // depend on the group it is in, so results are bitwise the same. The down
-    // projection is the residual GEMM, or split-K slabs + reduce when selected
-    // (the reference takes split-K at batch 1, lib.rs:218-225; here the
-    // residual GEMM is faster at batch 1 too, one launch instead of two per
-    // block, and keeps every image's result independent of the batch size).
-    // By default LayerNorm is folded
-    // into the QKV and gate/up GEMMs, fed by row statistics that the
-    // producers of x write (62 launches per group at b > 1); the unfused plan
-    // runs LayerNorm kernels as the reference does (86).
+    // one graph. The batch is cut into groups of images (see groups()) that
+    // run as independent chains, each over its own slice of every buffer: the
+    // kernels of one group fill the last, partial wave of workgroups of the
+    // other's. A row's arithmetic does not depend on the group it is in, so
+    // results are bitwise the same. The down projection is the residual GEMM,
+    // or split-K slabs + reduce when selected (the reference takes split-K at
+    // batch 1, lib.rs:218-225; here the residual GEMM is faster at batch 1
+    // too, one launch instead of two per block, and keeps every image's result
+    // independent of the batch size). By default LayerNorm is folded into the
+    // QKV and gate/up GEMMs, fed by row statistics that the producers of x
+    // write (62 launches per group at b > 1); the unfused plan runs LayerNorm
+    // kernels as the reference does (86).
     void prepare(uint64_t b, uint32_t slot = 0) {
         if (dhx_has_graph(engine_.get(), key(b, slot))) return;
         const uint32_t nb = groups(b);
@@ -499,9 +507,11 @@ public:
         if (ordered) dhx::engine_check(e, hipEventRecord(slot.last, stream), "hipEventRecord");
     }
 
-    // Number of image groups run side by side for a batch of b.
+    // Number of image groups run side by side for a batch of b: set_branches'
+    // count, or two from kTwoGroupRows on; groups of kMinBranchImages at least.
     uint32_t groups(uint64_t b) const {
-        return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(branches_, b / kMinBranchImages));
+        const uint64_t want = branches_ ? branches_ : b * tokens_ >= kTwoGroupRows ? 2 : 1;
+        return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, b / kMinBranchImages));
     }
 
     // Graph key: batch size plus one bit per plan variant.
@@ -524,7 +534,7 @@ private:
     uint64_t patches_ = 196, tokens_ = 201, tpad_ = 256, image_elems_ = 0;
     int splitk_ = 0;
     int fused_ln_ = 1;
-    uint32_t branches_ = 2;
+    uint32_t branches_ = 0;  // 0: not set, groups() chooses
     std::unique_ptr<dhx_engine, EngineFree> engine_;
     std::map<std::string, dhx_region> weights_;
     dhx_region a_[kBuffers];

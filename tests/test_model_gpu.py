@@ -266,6 +266,20 @@ def test_branches_are_bitwise_identical(models):
         m.set_branches(2)
 
 
+@pytest.mark.parametrize("images", [8, 23, 24, 31])
+def test_default_groups_on_both_sides_of_the_row_limit(weight_file, images):
+    # A model whose grouping was never set: one group below 4800 rows (23
+    # images of 201 tokens), two from there on, the same bits as either choice.
+    px = d.random_pixels(24, images)
+    with d.DINOv3.load(weight_file(1), d.Options(0, images)) as m:
+        out = m.forward(px)
+        launches = len(m.launch_timings(images, 1))
+        assert launches == 62 * (2 if images * 201 >= 4800 else 1)
+        for n in (1, 2):
+            m.set_branches(n)
+            assert np.array_equal(m.forward(px), out), f"{n} groups"
+
+
 def test_splitk_variant(models):
     # Both down-projection variants at batch 8 and at batch 1 (the
     # reference's split-K case, lib.rs:218-225): the same result to f16
