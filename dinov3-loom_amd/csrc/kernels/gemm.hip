@@ -28,7 +28,7 @@ using ResidTile = Tile<128, 64, 4, 1>;
 using ResidTileK = Tile<128, 64, 4, 1, 128>;  // down projection (k = 1536)
 using SwigluTile = Tile<256, 128, 4, 1, 64>;
 // SwiGLU for launches of fewer rows (batch 32's and 512x512 batch 8's image
-// groups of 3216 and 4116 rows, small batches): 128-row tiles, three
+// groups of 3216 and 4116 rows; below 2048 the rings): 128-row tiles, three
 // workgroups per CU instead of two. Measured in the two-group forward: the
 // 128-row tiles win at 3216 and 4116 rows (at 4116 the 256-row tiling's
 // last tile holds 20 rows), the 256-row ones at 6432 (batch 64's groups).
@@ -185,8 +185,8 @@ static hipError_t launch_swiglu_ring(const SwigluArgs& a, hipStream_t s) {
 // overlap one tile's epilogue with another's K loop, which the rings, taking
 // most of a CU's LDS, do not.
 //
-// For the larger launches, the XCD split (each XCD's L2 keeps 1/NS of the weights): two N slices for
-// the whole batch-64 launch, four for the image groups of 5120 - 8191 rows
+// For the larger launches, the XCD split (each XCD's L2 keeps 1/NS of the
+// weights): two N slices for the whole batch-64 launch, four for the image groups of 5120 - 8191 rows
 // that the forward runs concurrently (measured: forward +0.9 % at batch 64,
 // the whole-batch launch 2 % slower with four).
 hipError_t launch_swiglu(const SwigluArgs& a, hipStream_t s) {
