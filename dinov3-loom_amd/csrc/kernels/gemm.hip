@@ -66,6 +66,13 @@ hipError_t launch(Kernel kernel, int tiles, const Args& a, hipStream_t s) {
 }  // namespace
 
 hipError_t launch_patch_embed(const PatchEmbedArgs& a, hipStream_t s) {
+    const int ring = (a.images * a.grid * a.grid + gemm::kPatchRingRows - 1) / gemm::kPatchRingRows *
+                     (kHidden / gemm::kPatchRingCols);
+    if (ring <= kRound) {
+        const dim3 grid(gemm::tile_grid(ring)), block(128);
+        return a.stats ? start(gemm::patch_ring_kernel<true>, grid, block, 0, s, a)
+                       : start(gemm::patch_ring_kernel<false>, grid, block, 0, s, a);
+    }
     const int tiles = tiles_for<PatchTile>(a.images * a.grid * a.grid, kHidden);
     return a.stats ? launch<PatchTile>(gemm::patch_embed_kernel<PatchTile, true>, tiles, a, s)
                    : launch<PatchTile>(gemm::patch_embed_kernel<PatchTile, false>, tiles, a, s);

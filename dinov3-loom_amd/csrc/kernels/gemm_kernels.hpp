@@ -69,6 +69,52 @@ __device__ __forceinline__ void pair_stats(float* stats, size_t m, int slot, con
     if (store && hi == 0) *(float2_t*)(stats + m * kStatFloats + slot * 2) = float2_t{mean, q};
 }
 
+// A wave's 32 x 64 block of patch rows m_base .., rounded to f16 in LDS (st,
+// of pitch sp halfs), written to x as fragment pieces; with STATS also its
+// statistics slot.
+template <bool STATS>
+__device__ __forceinline__ void patch_rows(const PatchEmbedArgs& p, const half_t* st, int sp, int m_base, int n_base, int M,
+                                           int P) {
+    const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
+    const int m = m_base + l32;
+    const bool valid = m < M;
+    const size_t row = valid ? (size_t)m + (size_t)(m / P + 1) * kPrefix : 0;  // image*Tok + kPrefix + patch
+    // The wave's 32 patch rows land in x rows row(m_base) .. at most
+    // 32 + 5 * (32 / P + 1) rows further: within 8 row blocks.
+    const size_t rb0 = ((size_t)m_base + (size_t)(m_base / P + 1) * kPrefix) / 32;
+    const WtOut xo(p.x + rb0 * (kHidden / 16) * 512, 8 * (kHidden / 16) * 1024);
+    float v[32];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        const half8_t h = *(const half8_t*)(st + l32 * sp + ks * 16 + hi * 8);
+        if (valid)
+            xo.store((uint32_t)(frag_piece((int)row, n_base + ks * 16 + hi * 8, kHidden) - rb0 * (kHidden / 16) * 512) * 2, h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[ks * 8 + e] = (float)h[e];
+    }
+    if constexpr (STATS) pair_stats(p.stats, row, n_base / 64, v, hi, valid);
+}
+
+// CLS + registers, columns n0 .. n0 + BN - 1, of every image whose first patch
+// row lies in m0 .. m_end - 1, by threads tid of THREADS.
+template <int BN, int THREADS, bool STATS>
+__device__ __forceinline__ void patch_prefix(const PatchEmbedArgs& p, int tid, int m0, int m_end, int n0, int P, int Tok) {
+    for (int img = (m0 + P - 1) / P; img * P < m_end; ++img) {
+        for (int idx = tid; idx < kPrefix * BN; idx += THREADS) {
+            const int r = idx / BN, col = n0 + idx % BN;
+            p.x[frag_piece(img * Tok + r, col & ~7, kHidden) + (col & 7)] = (half_t)p.prefix[r * kHidden + col];
+        }
+        if constexpr (STATS) {
+            constexpr int slots = BN / 64;
+            for (int idx = tid; idx < kPrefix * slots * 2; idx += THREADS) {
+                const int r = idx / (slots * 2), e = idx % (slots * 2);
+                const int off = (n0 / 64) * 2 + e;
+                p.stats[((size_t)img * Tok + r) * kStatFloats + off] = p.prefix_stats[r * kStatFloats + off];
+            }
+        }
+    }
+}
+
 // Patch embedding + CLS/register scatter into the f16 residual stream x
 // (fragment order; with STATS, also the LayerNorm row statistics of x). Each
 // wave rounds its 32 x 64 block to f16 into LDS, then writes it as fragment
@@ -97,40 +143,111 @@ __global__ __launch_bounds__(T::THREADS) void patch_embed_kernel(DHX_PATCH_PARAM
                 *(half4_t*)(st + f.l32 * SP + (n - f.n_base)) = to_half4(group4(acc.v[i][0], g) + b);
             }
         wave_lds_sync();
-        const int m = f.m_base + f.l32;
-        const bool valid = m < M;
-        const size_t row = valid ? (size_t)m + (size_t)(m / P + 1) * kPrefix : 0;  // image*Tok + kPrefix + patch
-        // The wave's 32 patch rows land in x rows row(m_base) .. at most
-        // 32 + 5 * (32 / P + 1) rows further: within 8 row blocks.
-        const size_t rb0 = ((size_t)f.m_base + (size_t)(f.m_base / P + 1) * kPrefix) / 32;
-        const WtOut xo(p.x + rb0 * (kHidden / 16) * 512, 8 * (kHidden / 16) * 1024);
-        float v[32];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const half8_t h = *(const half8_t*)(st + f.l32 * SP + ks * 16 + f.hi * 8);
-            if (valid)
-                xo.store((uint32_t)(frag_piece((int)row, f.n_base + ks * 16 + f.hi * 8, kHidden) - rb0 * (kHidden / 16) * 512) * 2, h);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[ks * 8 + e] = (float)h[e];
-        }
-        if constexpr (STATS) pair_stats(p.stats, row, f.n_base / 64, v, f.hi, valid);
-        // CLS + registers of every image whose first patch row lies in this tile.
-        const int m_end = min(m0 + T::BM, M);
-        for (int img = (m0 + P - 1) / P; img * P < m_end; ++img) {
-            for (int idx = threadIdx.x; idx < kPrefix * T::BN; idx += T::THREADS) {
-                const int r = idx / T::BN, col = n0 + idx % T::BN;
-                p.x[frag_piece(img * Tok + r, col & ~7, kHidden) + (col & 7)] = (half_t)p.prefix[r * kHidden + col];
-            }
-            if constexpr (STATS) {
-                constexpr int slots = T::BN / 64;
-                for (int idx = threadIdx.x; idx < kPrefix * slots * 2; idx += T::THREADS) {
-                    const int r = idx / (slots * 2), e = idx % (slots * 2);
-                    const int off = (n0 / 64) * 2 + e;
-                    p.stats[((size_t)img * Tok + r) * kStatFloats + off] = p.prefix_stats[r * kStatFloats + off];
-                }
-            }
-        }
+        patch_rows<STATS>(p, st, SP, f.m_base, f.n_base, M, P);
+        patch_prefix<T::BN, T::THREADS, STATS>(p, threadIdx.x, m0, min(m0 + T::BM, M), n0, P, Tok);
     });
+}
+
+// Patch embedding for launches that one round of workgroups covers (see the
+// launcher): 32x64 tiles of two waves (one column block each) and a ring of
+// eight 64-deep stages, pixels as they are (float32) and weights, both by DMA.
+// patch_embed_kernel's twelve steps wait for loads issued one step ahead, on
+// 12 workgroups at 196 patches; here seven stages are in flight on 42:
+// alone at 196 patches 8.4 -> 5.6 us, at 1176 8.6 -> 6.0, and 3 us less of
+// the forward at one image. Left are the launch, one cold load, twelve barriers
+// and the stores. A stage holds four pixel rows of one channel of 32 patches as [row][patch]
+// [16 pixels], 16-byte chunk c of patch r at slot c ^ (r / 4) % 4, and 64
+// weight rows of 64 columns, chunk c of row r at slot c ^ (r / 2) % 8, so that
+// 16 consecutive rows' reads of one chunk cover all banks. The same MFMAs in
+// the same order as patch_embed_kernel: a row's result is bitwise the same.
+// Offsets into the pixels are 32 bits: the launcher bounds the launch.
+constexpr int kPatchRing = 8, kPatchRingRows = 32, kPatchRingCols = 64;
+constexpr int kPatchRingW = 32 * 64 * 2;  // halfs of a stage's pixels, after which its weights follow
+constexpr int kPatchRingHalfs = kPatchRingW + 64 * 64;
+
+// The K loop of one tile; see gemm_main_ring for the waits.
+__device__ __forceinline__ void patch_ring(const PatchEmbedArgs& p, half_t* const (&bufs)[kPatchRing], int m0, int n0, int M,
+                                           int P, float16_t& acc) {
+    constexpr int KT = 768 / 64;
+    const int S = 16 * p.grid;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hi = lane >> 5;
+    const __amdgpu_buffer_rsrc_t rp = dma_src(p.pixels, p.images * 3 * S * S * 4);
+    const __amdgpu_buffer_rsrc_t rw = dma_src(p.w + (size_t)n0 * 768, kPatchRingCols * 768 * 2);
+    // Each wave moves two of a stage's four pixel rows (16 patches a load) and
+    // 32 of its 64 weight rows (8 a load).
+    int ap[2], aw[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int m = min(m0 + 16 * h + (lane >> 2), M - 1);  // rows past M feed unstored outputs
+        const int img = m / P, q = m - img * P, gy = q / p.grid, gx = q - gy * p.grid;
+        ap[h] = ((img * 3 * S + gy * 16) * S + gx * 16) * 4 + ((lane & 3) ^ (lane >> 4)) * 16;
+        aw[h] = (lane >> 3) * 1536 + ((lane & 7) ^ (4 * h + (lane >> 4))) * 16;
+    }
+    auto lds = [](half_t* a) { return (__attribute__((address_space(3))) void*)a; };
+    auto load = [&](half_t* stage, int kt) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int dy = wave * 2 + (j >> 1);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, lds(stage + (dy * 2 + (j & 1)) * 512), 16, ap[j & 1],
+                                                     ((kt >> 2) * S + (kt & 3) * 4 + dy) * S * 4, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, lds(stage + kPatchRingW + (wave * 4 + j) * 512), 16, aw[j & 1],
+                                                     (wave * 4 + j) * 8 * 1536 + kt * 128, 0, 0);
+    };
+    acc = float16_t{};
+    static_for<kPatchRing - 1>([&](auto I) { load(bufs[decltype(I)::value], decltype(I)::value); });
+    static_for<KT>([&](auto I) {
+        constexpr int s = decltype(I)::value;
+        constexpr int ahead = KT - 1 - s < kPatchRing - 2 ? KT - 1 - s : kPatchRing - 2;  // later stages in flight
+        vm_barrier<ahead * 8>();
+        if constexpr (s + kPatchRing - 1 < KT) load(bufs[(s + kPatchRing - 1) % kPatchRing], s + kPatchRing - 1);
+        const half_t* const stage = bufs[s % kPatchRing];
+        const float* const a = (const float*)stage + l32 * 16;
+        const half_t* const w = stage + kPatchRingW + (wave * 32 + l32) * 64;
+        half8_t af[4], wf[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const half4_t lo = to_half4(*(const float4_t*)(a + kk * 512 + ((2 * hi) ^ ((l32 >> 2) & 3)) * 4));
+            const half4_t up = to_half4(*(const float4_t*)(a + kk * 512 + ((2 * hi + 1) ^ ((l32 >> 2) & 3)) * 4));
+            af[kk] = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
+            wf[kk] = *(const half8_t*)(w + ((2 * kk + hi) ^ ((l32 >> 1) & 7)) * 8);
+        }
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) acc = mfma32x32x16(wf[kk], af[kk], acc);
+    });
+}
+
+template <bool STATS>
+__global__ __launch_bounds__(128, 1) void patch_ring_kernel(DHX_PATCH_PARAMS) {
+    const PatchEmbedArgs p{pixels_, w_, bias_, prefix_, x_, images_, grid_, prefix_stats_, stats_};
+    constexpr int NT = kHidden / kPatchRingCols, SP = kPatchRingCols + 8;
+    __shared__ __attribute__((aligned(16))) half_t ring0[kPatchRingHalfs], ring1[kPatchRingHalfs], ring2[kPatchRingHalfs],
+        ring3[kPatchRingHalfs], ring4[kPatchRingHalfs], ring5[kPatchRingHalfs], ring6[kPatchRingHalfs],
+        ring7[kPatchRingHalfs];
+    __shared__ __attribute__((aligned(16))) half_t st[32 * SP];
+    __shared__ __attribute__((aligned(16))) float bias[dma_copy_bytes(kPatchRingCols * 4) / 4];
+    half_t* const bufs[kPatchRing] = {ring0, ring1, ring2, ring3, ring4, ring5, ring6, ring7};
+    const int P = p.grid * p.grid, M = p.images * P;
+    const int t = xcd_tile(NT * ((M + kPatchRingRows - 1) / kPatchRingRows));
+    if (t < 0) return;  // uniform per workgroup
+    const int n0 = (t % NT) * kPatchRingCols, m0 = (t / NT) * kPatchRingRows;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    dma_copy<kPatchRingCols * 4, 2>(dma_src(p.bias + n0, kPatchRingCols * 4), bias, tid);
+    float16_t acc;
+    patch_ring(p, bufs, m0, n0, M, P, acc);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const int n = wave * 32 + g * 8 + (lane >> 5) * 4;
+        *(half4_t*)(st + (lane & 31) * SP + n) = to_half4(group4(acc, g) + *(const float4_t*)&bias[n]);
+    }
+    lds_barrier();
+    if (wave == 0)
+        patch_rows<STATS>(p, st, SP, m0, n0, M, P);
+    else
+        patch_prefix<kPatchRingCols, 64, STATS>(p, lane, m0, min(m0 + kPatchRingRows, M), n0, P, P + kPrefix);
 }
 
 template <class T>

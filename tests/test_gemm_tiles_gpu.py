@@ -8,7 +8,7 @@ import pytest
 
 import oracle
 
-from test_kernels_gpu import (K_QKV, K_QKV_LN, K_RESID, K_RESID_S, K_SWIGLU, K_SWIGLU_LN, _keys, allocf, eng,  # noqa: F401
+from test_kernels_gpu import (K_PATCH, K_PATCH_S, K_QKV, K_QKV_LN, K_RESID, K_RESID_S, K_SWIGLU, K_SWIGLU_LN, _keys, allocf, eng,  # noqa: F401
                               f16, read_heads, readf, slot_stats, up, upf)
 
 pytestmark = pytest.mark.gpu
@@ -98,3 +98,28 @@ def test_swiglu_rows_do_not_depend_on_the_tile(eng):  # noqa: F811
     for rows in (1, 33, 640, 641, 1280, 1281, 2048, 2049, 5119, 5120):
         for name, g, r in zip(("plain", "LN"), launch(rows), want):
             assert np.array_equal(g, r[:rows]), (rows, name)
+
+
+@pytest.mark.parametrize("grid,most,counts", [(1, 1400, (1, 31, 33, 1344, 1345)), (3, 160, (1, 4, 149, 150)),
+                                              (14, 8, (1, 3, 6, 7)), (37, 2, (1,))])
+def test_patch_rows_do_not_depend_on_the_tile(eng, grid, most, counts):  # noqa: F811
+    rng = np.random.default_rng(grid)
+    T, S = grid * grid + 5, 16 * grid
+    px = rng.normal(size=(most, 3, S, S)).astype(np.float32)
+    w = up(eng, f16(rng.normal(size=(384, 768)) * 0.02))
+    b, prefix = up(eng, rng.normal(size=384).astype(np.float32)), up(eng, rng.normal(size=(5, 384)).astype(np.float32))
+    pstats = up(eng, rng.normal(size=(5, 12)).astype(np.float32))
+
+    def launch(images):
+        p, x, xs, st = up(eng, px[:images]), *(allocf(eng, images * T, 384) for _ in range(2)), eng.allocate(images * T * 48)
+        run(eng, K_PATCH, [images, grid], [p, w, b, prefix, x])
+        run(eng, K_PATCH_S, [images, grid], [p, w, b, prefix, pstats, xs, st])
+        y = readf(eng, x, images * T, 384)
+        assert np.array_equal(readf(eng, xs, images * T, 384), y)
+        return y, eng.read(st, np.float32, (images * T, 12))
+
+    want, want_stats = launch(most)
+    for images in counts:
+        got, stats = launch(images)
+        assert np.array_equal(got, want[:images * T]), images
+        assert np.array_equal(stats, want_stats[:images * T]), images
