@@ -391,6 +391,31 @@ void engine_wait_readback(dhx_engine* e, uint32_t slot) {
     hip_check(e, hipEventSynchronize(e->out_done[slot]), "readback wait");
 }
 
+void engine_run_chunk(dhx_engine* e, dhx_region dst, uint64_t in_bytes, uint64_t graph, dhx_region src, uint64_t out_bytes,
+                      uint32_t slot) {
+    ensure_usable(e);
+    check_slot(e, slot);
+    check_region(e, dst);
+    check_region(e, src);
+    if (in_bytes > dst.bytes) throw Error("input exceeds allocated region");
+    if (in_bytes > e->pin_in_bytes) throw Error("input exceeds reserved staging");
+    if (out_bytes > src.bytes) throw Error("output exceeds allocated region");
+    if (out_bytes > e->pin_out_bytes) throw Error("output exceeds reserved staging");
+    auto it = e->graphs.find(graph);
+    if (it == e->graphs.end()) throw Error("batch has not been prepared");
+    set_device(e);
+    // Transfers queued for the slot through the other streams come first; all
+    // that is queued here is done on return, so the slot's events stay as they
+    // are. The other graphs that read dst run on this stream too.
+    hip_check(e, hipEventSynchronize(e->in_done[slot]), "upload wait");
+    hip_check(e, hipEventSynchronize(e->out_done[slot]), "readback wait");
+    hip_check(e, hipMemcpyAsync(region_ptr(e, dst), e->pin_in[slot], in_bytes, hipMemcpyHostToDevice, e->stream), "upload");
+    hip_check(e, hipGraphLaunch(it->second.exec, e->stream), "graph launch");
+    hip_check(e, hipMemcpyAsync(e->pin_out[slot], region_ptr(e, src), out_bytes, hipMemcpyDeviceToHost, e->stream),
+              "readback copy");
+    hip_check(e, hipStreamSynchronize(e->stream), "synchronize");
+}
+
 hipStream_t engine_stream(const dhx_engine* e) { return e->stream; }
 
 int engine_device(const dhx_engine* e) { return e->device; }

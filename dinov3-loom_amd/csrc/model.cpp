@@ -248,11 +248,12 @@ public:
 
     // lib.rs:90-114: chunks of max_batch images, pipelined over the two
     // transfer slots: chunk i uses slot i % 2. This thread issues every HIP
-    // call (uploads, graph launches, readbacks); with more than one chunk a
-    // Copier thread does the host copies into and out of the pinned staging
-    // buffers, each handed over as soon as its buffer is free: chunk i+1's
-    // input copy and chunk i-1's output copy run while chunk i is launched
-    // and computed. Results are those of the chunks run one at a time.
+    // call (uploads, graph launches, readbacks) while a Copier thread does the
+    // host copies into and out of the pinned staging buffers, each handed over
+    // as soon as its buffer is free: chunk i+1's input copy and chunk i-1's
+    // output copy run while chunk i is launched and computed. A single chunk
+    // has nothing to overlap and runs on one stream. Results are those of the
+    // chunks run one at a time.
     void forward(const float* pixels, uint64_t n, float* out, uint64_t out_floats) {
         check_input(pixels, n);
         const uint64_t batch = n / image_elems_;
@@ -268,8 +269,15 @@ public:
         auto out_bytes = [&](uint64_t i) { return size_of(i) * per_image * 4; };
         if (in_bytes(0) > dhx::engine_staging_in_bytes(e) || out_bytes(0) > dhx::engine_staging_out_bytes(e))
             throw Error("chunk exceeds reserved staging");
+        if (chunks == 1) {
+            dhx::engine_wait_upload(e, 0);  // staging buffer free
+            dhx::parallel_copy(dhx::engine_staging_in(e, 0), pixels, in_bytes(0));
+            dhx::engine_run_chunk(e, a_[image_buffer(0)], in_bytes(0), key(batch, 0), a_[out_buffer(0)], out_bytes(0), 0);
+            dhx::parallel_copy(out, dhx::engine_staging_out(e, 0), out_bytes(0));
+            return;
+        }
         std::vector<uint64_t> filled(chunks), drained(chunks);
-        Copier copier(chunks > 1);
+        Copier copier(true);
         // Chunk i's pixels into slot i % 2's input staging, once the slot's
         // previous upload has left it.
         auto fill = [&](uint64_t i) {
@@ -287,7 +295,7 @@ public:
                                        out_bytes(i));
         };
         fill(0);
-        if (chunks > 1) fill(1);
+        fill(1);
         for (uint64_t i = 0; i < chunks; ++i) {
             const uint32_t slot = (uint32_t)(i & 1);
             copier.wait(filled[i]);
