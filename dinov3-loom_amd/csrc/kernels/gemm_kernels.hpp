@@ -359,7 +359,8 @@ __device__ __forceinline__ void qkv_epilogue(const QkvArgs& p, const Acc<T>& acc
                     w_up = *(const float4_t*)&wsum[nl + 32];
                 }
                 // Explicit FMAs: a row's result is the same on every tile
-                // shape, however the compiler would contract each.
+                // shape, however the compiler would contract each. lo's
+                // products are the fused ones in both outputs.
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     if constexpr (LN) {
@@ -371,7 +372,7 @@ __device__ __forceinline__ void qkv_epilogue(const QkvArgs& p, const Acc<T>& acc
                     }
                     const float l = lo[e];
                     lo[e] = fmaf(l, co[g][e], -(up[e] * si[g][e]));  // x[c] cos - x[c+32] sin
-                    up[e] = fmaf(up[e], co[g][e], l * si[g][e]);     // x[c+32] cos + x[c] sin
+                    up[e] = fmaf(l, si[g][e], up[e] * co[g][e]);     // x[c+32] cos + x[c] sin
                 }
                 lo_h[g] = to_half4(lo);
                 up_h[g] = to_half4(up);

@@ -123,3 +123,28 @@ def test_patch_rows_do_not_depend_on_the_tile(eng, grid, most, counts):  # noqa:
         got, stats = launch(images)
         assert np.array_equal(got, want[:images * T]), images
         assert np.array_equal(stats, want_stats[:images * T]), images
+
+
+@pytest.mark.parametrize("images", [1, 26])
+def test_qkv_rotation_rounds_the_second_halfs_product(eng, images):  # noqa: F811
+    # Identity weights and no bias, so the sums are the inputs and the outputs
+    # show the rotation's own rounding: of lo cos - up sin and up cos + lo sin
+    # the products with up are rounded to float32, those with lo are fused, and the
+    # sum is rounded once, to float16.
+    grid, T, tpad = 14, 201, 256
+    rng = np.random.default_rng(images)
+    x = f16(rng.normal(size=(images * T, 384)))
+    w = upf(eng, f16(np.tile(np.eye(384), (3, 1))))
+    cos, sin = oracle.rope_tables(grid)
+    nb = images * 6 * tpad * 64 * 2
+    out = [eng.allocate(nb) for _ in range(3)]
+    run(eng, K_QKV, [images, grid, tpad], [upf(eng, x), w, up(eng, np.zeros(1152, np.float32)), up(eng, cos), up(eng, sin)] + out)
+    h = x.reshape(images, T, 6, 64).transpose(0, 2, 1, 3).astype(np.float64)
+    lo, hi = h[:, :, 5:, :32], h[:, :, 5:, 32:]
+    c, s = (t[:, :32].astype(np.float64) for t in (cos, sin))
+    want = h.copy()
+    want[:, :, 5:, :32] = lo * c - (hi * s).astype(np.float32)
+    want[:, :, 5:, 32:] = lo * s + (hi * c).astype(np.float32)
+    for r, ref in zip(out, (want, want, h)):
+        got, ref = read_heads(eng, r, images, tpad)[:, :, :T], ref.astype(np.float16)
+        assert np.array_equal(got, ref), f"{int((got != ref).sum())} of {ref.size} differ"
