@@ -203,7 +203,7 @@ __device__ __forceinline__ void attend32(QueryState& st, const half_t* sK, const
     // inside f16.
     float p[16], sum;
     if constexpr (FIRST) {
-        st.m_run = block_max32(s);
+        st.m_run = fmaxf(block_max32(s), st.m_run);  // as below, also for a block whose scores are all -inf
         sum = weights32(s, st.m_run, p);
     } else {
         sum = weights32(s, st.m_run, p);
@@ -473,7 +473,7 @@ __device__ __forceinline__ void parallel_blocks(const AttentionArgs& p, half_t* 
     for (int kk = 0; kk < 4; ++kk) st.qf[kk] = *(const half8_t*)(sq + kk * 512 + lane * 8) * (half_t)0.125f;
     float16_t s = scores32(k_own, st.qf, at);
     mask32(s, wave * 32, T, hi);
-    if (wave == 0) smax[l32] = block_max32(s);  // both lanes of a pair hold the pair's
+    if (wave == 0) smax[l32] = fmaxf(block_max32(s), st.m_run);  // both lanes of a pair hold the pair's
     vm_barrier<0>();
     float w[16];
     const float sum = weights32(s, smax[l32], w);

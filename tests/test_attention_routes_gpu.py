@@ -66,3 +66,35 @@ def test_edges_match_the_oracle(eng, grid, scale):  # noqa: F811
         rows = slice(i * T, (i + 1) * T)
         want = oracle.attention(*(m[rows].astype(np.float64) for m in (q, k, v)))
         check(got[rows], want, atol=2.0**-9 * np.abs(v[rows].astype(np.float64)).max(), what=f"T={T} image {i}")
+
+
+# Scores of -inf over the whole first key block (keys 0..31) and one later one:
+# the softmax runs over the other keys, whichever kernel takes the launch.
+@pytest.mark.parametrize("grid,images,most", [(8, 1, 20), (14, 6, 10), (16, 4, 8), (21, 3, 6), (22, 5, 8), (32, 2, 6)])
+def test_first_block_of_minus_infinities(eng, grid, images, most):  # noqa: F811
+    q, k, v = inputs(grid, most)
+    T = grid * grid + 5
+    q[:, ::64] = np.abs(q[:, ::64]) + np.float16(0.5)
+    k.reshape(most, T, 384)[:, :32, ::64] = -np.inf
+    k.reshape(most, T, 384)[:, 40, ::64] = -np.inf
+    want = launch(eng, [q, k, v], most, grid)
+    got = launch(eng, [q, k, v], images, grid)
+    assert np.array_equal(got, want[:images * T])
+    r = slice(0, T)
+    ref = oracle.attention(*(m[r].astype(np.float64) for m in (q, k, v)))
+    check(got[r], ref, atol=2.0**-9 * np.abs(v[r].astype(np.float64)).max(), what=f"T={T}")
+
+
+# A score of +inf or NaN, or a NaN value, makes its query's (its key's) outputs
+# NaN, the same ones on every kernel.
+@pytest.mark.parametrize("key", [3, 37])
+@pytest.mark.parametrize("what", ["k=+inf", "k=nan", "v=nan"])
+@pytest.mark.parametrize("grid,images,most", [(8, 1, 20), (14, 6, 10), (16, 4, 8), (22, 5, 8), (32, 2, 6)])
+def test_infinities_and_nan_do_not_depend_on_the_launch(eng, grid, images, most, what, key):  # noqa: F811
+    q, k, v = inputs(grid, most)
+    T = grid * grid + 5
+    (k if what[0] == "k" else v).reshape(most, T, 384)[:, key, :2] = np.inf if "inf" in what else np.nan
+    want = launch(eng, [q, k, v], most, grid)
+    got = launch(eng, [q, k, v], images, grid)
+    assert np.isnan(got).any() and not np.isnan(got).all()
+    assert np.array_equal(got, want[:images * T], equal_nan=True)
