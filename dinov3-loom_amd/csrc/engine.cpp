@@ -207,14 +207,16 @@ hipError_t launch_one(dhx_engine* e, const dhx_launch& l, hipStream_t stream, bo
         case DHX_K_LAYERNORM_F32:
             return launch_layernorm({Hf(0), F(1), F(2), P(3), (int)s[0], l.kernel == DHX_K_LAYERNORM_F32}, stream);
         case DHX_K_QKV_ROPE:
-            return launch_qkv_rope({Hf(0), Hf(1), F(2), F(3), F(4), Hf(5), Hf(6), Hf(7), (int)s[0], (int)s[1], (int)s[2]},
+            return launch_qkv_rope({Hf(0), Hf(1), F(2), F(3), F(4), Hf(5), Hf(6), Hf(7), (int)s[0], (int)s[1], (int)s[2],
+                                    nullptr, nullptr, shared},
                                    stream);
         case DHX_K_QKV_ROPE_LN:
             return launch_qkv_rope({Hf(0), Hf(2), F(4), F(5), F(6), Hf(7), Hf(8), Hf(9), (int)s[0], (int)s[1], (int)s[2],
-                                    F(1), F(3)},
+                                    F(1), F(3), shared},
                                    stream);
         case DHX_K_ATTENTION:
-            return launch_attention({Hf(0), Hf(1), Hf(2), Hf(3), (int)s[0], (int)tokens_for(s[1]), (int)s[2]}, stream);
+            return launch_attention({Hf(0), Hf(1), Hf(2), Hf(3), (int)s[0], (int)tokens_for(s[1]), (int)s[2], shared},
+                                    stream);
         case DHX_K_RESID:
             return launch_resid({Hf(0), Hf(1), F(2), F(3), Hf(4), (int)s[0], (int)s[1], nullptr, shared}, stream);
         case DHX_K_RESID_STATS:

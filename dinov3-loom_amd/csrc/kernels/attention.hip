@@ -726,7 +726,11 @@ hipError_t launch_split(const AttentionArgs& a, int groups, hipStream_t s) {
 // -> 1800; equal to attention_kernel from 581 tokens on, 5 % slower at 405).
 // 512x512 (17 blocks per half) in more than one round takes the unrolled walk
 // (batch 8 975 -> 964 us); in one round its 80 KB of code cost more to fetch
-// than they save (batch 1 449 against 424, batch 4 636 against 629). 201
+// than they save (batch 1 449 against 424, batch 4 636 against 629). Beside
+// another image group's kernels (a.shared) there are CUs to share and code to
+// fetch once for both: batch 8 in two groups 1005 -> 985 us unrolled, and 128
+// queries are the better workgroup (two groups, 64 -> 128: 352x352 batch 10
+// 684 -> 659 us, 400x400 batch 8 720 -> 684). 201
 // tokens: seven blocks of 32 keys, unrolled. Otherwise blocks of 64 keys with
 // a run-time count.
 hipError_t launch_attention(const AttentionArgs& a, hipStream_t s) {
@@ -737,8 +741,8 @@ hipError_t launch_attention(const AttentionArgs& a, hipStream_t s) {
     const int total32 = nkb * kHeads * a.images;
     if (nkb <= kMaxParallel && total32 <= kRound) return launch_parallel<kMaxParallel>(a, nkb, total32, s);
     if (nkb >= kSplitBlocks) {
-        if (total64 <= kRound) return launch_split<0, 2>(a, total64, s);
-        if ((nkb + 1) / 2 == 17 && total > kRound) return launch_split<17, 4>(a, total, s);
+        if ((nkb + 1) / 2 == 17 && (a.shared || total > kRound)) return launch_split<17, 4>(a, total, s);
+        if (!a.shared && total64 <= kRound) return launch_split<0, 2>(a, total64, s);
         return launch_split<0, 4>(a, total, s);
     }
     return nkb == 7 ? start(attention_kernel<7>, grid, block, 0, s, a) : start(attention_kernel<0>, grid, block, 0, s, a);

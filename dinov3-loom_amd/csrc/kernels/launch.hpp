@@ -73,6 +73,9 @@ struct QkvArgs {
     int tpad;
     const float* stats = nullptr;
     const float* wsum = nullptr;
+    // Other kernels run beside this launch (concurrent image groups); chooses
+    // the tile shape only, not the result.
+    bool shared = false;
 };
 
 // softmax(q k^T / 8) v per (image, head) over that image's T tokens, with
@@ -87,6 +90,7 @@ struct AttentionArgs {
     int images;
     int tokens;
     int tpad;
+    bool shared = false;  // as in QkvArgs
 };
 
 // x[rows][384] += ls * (a[rows][k] . W[384][k]^T + b), f16 residual in place
@@ -100,9 +104,7 @@ struct ResidArgs {
     int rows;
     int k;
     float* stats = nullptr;  // optional: row statistics of the updated x
-    // Other kernels run beside this launch (concurrent image groups); chooses
-    // the tile shape only, not the result.
-    bool shared = false;
+    bool shared = false;     // as in QkvArgs
 };
 
 // act[rows][1536] frag = silu(h.Wg^T + bg) * (h.Wu^T + bu), h frag; W and b are packed

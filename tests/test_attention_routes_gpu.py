@@ -8,17 +8,24 @@ import pytest
 
 import oracle
 
-from test_kernels_gpu import K_ATTN, allocf, check, eng, f16, heads_frag, readf, run, up  # noqa: F401
+from test_kernels_gpu import K_ATTN, _keys, allocf, check, eng, f16, heads_frag, readf, run, up  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
 
-def launch(e, mats, images, grid):
+def launch(e, mats, images, grid, beside=False):
     T = grid * grid + 5
     tpad = (T + 127) // 128 * 128
     ins = [up(e, heads_frag(m[:images * T], images, T, tpad)) for m in mats]
     out = allocf(e, images * T, 384)
-    run(e, K_ATTN, [images, grid, tpad], ins + [out])
+    if beside:  # one of two branches of a plan
+        key, other = next(_keys), allocf(e, images * T, 384)
+        e.record_branches(key, [[(K_ATTN, [images, grid, tpad], ins + [o])] for o in (out, other)])
+        e.replay(key)
+        e.synchronize()
+        assert np.array_equal(readf(e, other, images * T, 384), readf(e, out, images * T, 384), equal_nan=True)
+    else:
+        run(e, K_ATTN, [images, grid, tpad], ins + [out])
     return readf(e, out, images * T, 384)
 
 
@@ -49,8 +56,9 @@ def test_images_do_not_depend_on_the_launch(eng, grid, most, counts, ramp):  # n
     want = launch(eng, mats, most, grid)
     assert np.all(np.isfinite(want))
     for images in counts:
-        got = launch(eng, mats, images, grid)
-        assert np.array_equal(got, want[:images * T]), images
+        for beside in (False, True):
+            got = launch(eng, mats, images, grid, beside)
+            assert np.array_equal(got, want[:images * T]), (images, beside)
 
 
 @pytest.mark.parametrize("grid", [1, 5, 7, 21, 22, 25])
@@ -80,6 +88,7 @@ def test_first_block_of_minus_infinities(eng, grid, images, most):  # noqa: F811
     want = launch(eng, [q, k, v], most, grid)
     got = launch(eng, [q, k, v], images, grid)
     assert np.array_equal(got, want[:images * T])
+    assert np.array_equal(launch(eng, [q, k, v], images, grid, beside=True), got)
     r = slice(0, T)
     ref = oracle.attention(*(m[r].astype(np.float64) for m in (q, k, v)))
     check(got[r], ref, atol=2.0**-9 * np.abs(v[r].astype(np.float64)).max(), what=f"T={T}")
@@ -98,3 +107,4 @@ def test_infinities_and_nan_do_not_depend_on_the_launch(eng, grid, images, most,
     got = launch(eng, [q, k, v], images, grid)
     assert np.isnan(got).any() and not np.isnan(got).all()
     assert np.array_equal(got, want[:images * T], equal_nan=True)
+    assert np.array_equal(launch(eng, [q, k, v], images, grid, beside=True), got, equal_nan=True)
