@@ -57,6 +57,7 @@ using QkvRing64 = Tile<64, 64, 2, 1, 64>;
 using QkvRing64W = Tile<64, 128, 2, 2, 64>;
 using QkvRing128 = Tile<128, 128, 4, 2, 64>;
 constexpr int kRound = 256;  // workgroups of one per CU
+constexpr int kQkvSharedRing = 22 * 128;  // QkvRing128's most rows beside other kernels
 
 template <class T, class Kernel, class Args>
 hipError_t launch(Kernel kernel, int tiles, const Args& a, hipStream_t s) {
@@ -100,12 +101,16 @@ static hipError_t launch_qkv_ring(const QkvArgs& a, hipStream_t s) {
 // below / 64x64 / 64x128 / 128x128: 201 rows 418 / 390 / 395 / 405 us, 603
 // rows 426 / 401 / 406 / 420, 1005 rows 411 / 434 / 400 / 415, 1608 rows 446
 // / 461 / 427 / 440, 2412 rows 466 / 509 / 481 / 453, 3216 rows 503 / 586 /
-// 519 / 487, 4020 rows 513 / 645 / 583 / 559.
+// 519 / 487, 4020 rows 513 / 645 / 583 / 559. Beside another image group's
+// kernels the 128x128 ring, which takes most of a CU's LDS, only to 2816 rows
+// (two groups, the tiles below / 128x128: 2 x 2412 rows 590 / 578 us, 2 x 2610
+// 685 / 644, 2 x 2814 667 / 632; 2 x 2835 711 / 728, 2 x 3216 684 / 681, 2 x
+// 3240 739 / 768, 3393 and 3654 732 / 756).
 hipError_t launch_qkv_rope(const QkvArgs& a, hipStream_t s) {
     const int rows = a.images * (a.grid * a.grid + kPrefix);
     if (rows <= kRound / 18 * 64) return launch_qkv_ring<QkvRing64, 4>(a, s);
     if (rows <= kRound / 9 * 64) return launch_qkv_ring<QkvRing64W, 4>(a, s);
-    if (rows <= kRound / 9 * 128) return launch_qkv_ring<QkvRing128, 3>(a, s);
+    if (rows <= (a.shared ? kQkvSharedRing : kRound / 9 * 128)) return launch_qkv_ring<QkvRing128, 3>(a, s);
     return rows < kQkvSmallRows ? launch_qkv_tiles<QkvTileS>(a, s) : launch_qkv_tiles<QkvTile>(a, s);
 }
 

@@ -53,7 +53,7 @@ def test_resid_rows_do_not_depend_on_the_tile(eng, kdim):  # noqa: F811
             assert np.array_equal(stats, want_stats[:rows]), (rows, beside)
 
 
-@pytest.mark.parametrize("grid,most,counts", [(4, 300, (1, 2, 42, 43, 85, 86, 170, 171)), (14, 26, (1, 4, 5, 8, 9, 17, 18)),
+@pytest.mark.parametrize("grid,most,counts", [(4, 300, (1, 2, 42, 43, 85, 86, 170, 171)), (14, 26, (1, 4, 5, 8, 9, 14, 15, 17, 18)),
                                               (59, 2, (1,))])
 def test_qkv_rows_do_not_depend_on_the_tile(eng, grid, most, counts):  # noqa: F811
     rng = np.random.default_rng(grid)
@@ -64,19 +64,20 @@ def test_qkv_rows_do_not_depend_on_the_tile(eng, grid, most, counts):  # noqa: F
     wsum, b = (up(eng, (rng.normal(size=1152) * 0.1).astype(np.float32)) for _ in range(2))
     cos, sin = (up(eng, t) for t in oracle.rope_tables(grid))
 
-    def launch(images):
+    def launch(images, beside=False):
         xr, st, nb = upf(eng, x[:images * T]), up(eng, slot_stats(x[:images * T])), images * 6 * tpad * 64 * 2
         got = []
         for kernel, first in ((K_QKV, [xr, w, b]), (K_QKV_LN, [xr, st, w, wsum, b])):
-            out = [eng.allocate(nb) for _ in range(3)]
-            run(eng, kernel, [images, grid, tpad], first + [cos, sin] + out)
+            out, other = ([eng.allocate(nb) for _ in range(3)] for _ in range(2))
+            run(eng, kernel, [images, grid, tpad], first + [cos, sin] + out, first + [cos, sin] + other if beside else None)
             got += [read_heads(eng, r, images, tpad) for r in out]
         return got
 
     want = launch(most)
     for images in counts:
-        for name, g, r in zip(("q", "k", "v", "q LN", "k LN", "v LN"), launch(images), want):
-            assert np.array_equal(g, r[:images]), (images, name)
+        for beside in (False, True):
+            for name, g, r in zip(("q", "k", "v", "q LN", "k LN", "v LN"), launch(images, beside), want):
+                assert np.array_equal(g, r[:images]), (images, beside, name)
 
 
 def test_swiglu_rows_do_not_depend_on_the_tile(eng):  # noqa: F811
