@@ -728,11 +728,12 @@ hipError_t launch_split(const AttentionArgs& a, int groups, hipStream_t s) {
 // (batch 8 975 -> 964 us); in one round its 80 KB of code cost more to fetch
 // than they save (batch 1 449 against 424, batch 4 636 against 629). Beside
 // another image group's kernels (a.shared) there are CUs to share and code to
-// fetch once for both: batch 8 in two groups 1005 -> 985 us unrolled, and 128
-// queries are the better workgroup (two groups, 64 -> 128: 352x352 batch 10
-// 684 -> 659 us, 400x400 batch 8 720 -> 684). 201
-// tokens: seven blocks of 32 keys, unrolled. Otherwise blocks of 64 keys with
-// a run-time count.
+// fetch once for both: batch 8 in two groups 1005 -> 985 us unrolled, and 64
+// queries are the better workgroup to 192 of them only (two groups, 64 | 128:
+// 2 x 192 workgroups, 352x352 batch 8, 580 | 611 us; 216 and 270, 368x368
+// batch 9, 675 | 664; 2 x 240, 352x352 batch 10, 684 | 659, 400x400 batch 8,
+// 720 | 684). 201 tokens: seven blocks of 32 keys, unrolled. Otherwise blocks
+// of 64 keys with a run-time count.
 hipError_t launch_attention(const AttentionArgs& a, hipStream_t s) {
     const int nqb = (a.tokens + QB - 1) / QB, total = nqb * kHeads * a.images;
     const int total64 = (a.tokens + 63) / 64 * kHeads * a.images;
@@ -742,7 +743,7 @@ hipError_t launch_attention(const AttentionArgs& a, hipStream_t s) {
     if (nkb <= kMaxParallel && total32 <= kRound) return launch_parallel<kMaxParallel>(a, nkb, total32, s);
     if (nkb >= kSplitBlocks) {
         if ((nkb + 1) / 2 == 17 && (a.shared || total > kRound)) return launch_split<17, 4>(a, total, s);
-        if (!a.shared && total64 <= kRound) return launch_split<0, 2>(a, total64, s);
+        if (total64 <= (a.shared ? kRound * 3 / 4 : kRound)) return launch_split<0, 2>(a, total64, s);
         return launch_split<0, 4>(a, total, s);
     }
     return nkb == 7 ? start(attention_kernel<7>, grid, block, 0, s, a) : start(attention_kernel<0>, grid, block, 0, s, a);

@@ -40,7 +40,7 @@ def inputs(grid, images, scale=2.0):
 # and 19 blocks (64-query workgroups up to 256 of them), 1029 tokens (64
 # queries to 2 images, 128 from 3, the unrolled walk from 5), 2030 tokens.
 ROUTES = [(4, 50, (1, 42, 43)), (8, 20, (1, 14, 15)), (12, 12, (1, 8, 9)), (14, 10, (1, 6, 7)), (15, 8, (1, 5, 6)),
-          (16, 8, (1, 4, 5)), (21, 6, (1, 3, 4)), (22, 8, (1, 5, 6)), (24, 8, (1, 4, 5)), (32, 6, (1, 2, 3, 4, 5)),
+          (16, 8, (1, 4, 5)), (21, 6, (1, 3, 4)), (22, 8, (1, 4, 5, 6)), (24, 8, (1, 4, 5)), (32, 6, (1, 2, 3, 4, 5)),
           (45, 3, (1, 2))]
 
 
