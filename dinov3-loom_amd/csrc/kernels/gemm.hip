@@ -57,6 +57,7 @@ using QkvRing64 = Tile<64, 64, 2, 1, 64>;
 using QkvRing64W = Tile<64, 128, 2, 2, 64>;
 using QkvRing128 = Tile<128, 128, 4, 2, 64>;
 constexpr int kRound = 256;  // workgroups of one per CU
+constexpr int kResidRing128Rows = 5120;
 constexpr int kQkvSharedRing = 22 * 128;  // QkvRing128's most rows beside other kernels
 
 template <class T, class Kernel, class Args>
@@ -128,7 +129,9 @@ hipError_t launch_resid(const ResidArgs& a, hipStream_t s) {
     // (one chain, graph replay), against resid_kernel: o-projection 32x64 at
     // 201 rows 412 -> 403 us (64x64 406); down projection 64x64 at 201 / 1005
     // / 2412 rows 412 -> 376, 404 -> 368, 488 -> 455, at 3216 rows 528 -> 551;
-    // 128x64 there 528 -> 517 and at 4020 rows 539 -> 527. To 1344 rows the
+    // 128x64 there 528 -> 517, at 4020 rows 539 -> 527, at 5025 rows 563 ->
+    // 549, but not to the end of its round: 512x512 batch 5 (5145 rows) 803 ->
+    // 839 us, 384x384 batch 9 (5229 rows) 732 -> 753. To 1344 rows the
     // down projection's 32x64 tile with five 64-deep stages in flight takes
     // 8.5 us off each of these (201 rows 295.3 -> 286.8, 1005 rows 315.6 ->
     // 308.5; three or four 128-deep stages 294, 293, 1608 rows 355 -> 377).
@@ -142,7 +145,8 @@ hipError_t launch_resid(const ResidArgs& a, hipStream_t s) {
     const int round = a.rows <= kRound / 6 * 32   ? 32
                       : a.rows <= kRound / 6 * 64 ? 64
                       : a.shared                  ? 0
-                      : a.rows <= kRound / 6 * 128 ? 128
+                      : a.rows < kResidRing128Rows ? 128
+                      : a.rows <= kRound / 6 * 128 ? 0
                       : a.rows <= kRound / 3 * 128 ? 256 : 0;
     if (a.k == kHidden && round == 32) return launch_resid_ring<ResidRing32, 4, kHidden>(a, s);
     if (a.k == kHidden && round == 64) return launch_resid_ring<ResidRing64, 5, kHidden>(a, s);

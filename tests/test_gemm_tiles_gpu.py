@@ -46,7 +46,7 @@ def test_resid_rows_do_not_depend_on_the_tile(eng, kdim):  # noqa: F811
         return y, eng.read(st, np.float32, (rows, 12))
 
     want, want_stats = launch(most)
-    for rows in (1, 32, 33, 65, 1344, 1345, 2688, 2689, 5376, 5377, 10880, 10881):
+    for rows in (1, 32, 33, 65, 1344, 1345, 2688, 2689, 5119, 5120, 5376, 5377, 10880, 10881):
         for beside in (False, True):
             got, stats = launch(rows, beside)
             assert np.array_equal(got, want[:rows]), (rows, beside)
