@@ -157,9 +157,18 @@ constexpr uint64_t align256(uint64_t v) { return (v + 255) & ~255ull; }
 // every pixel first), split over host threads for large batches.
 bool all_finite(const float* p, uint64_t n) {
     auto scan = [p](uint64_t a, uint64_t b) {
-        bool ok = true;
-        for (uint64_t i = a; i < b; ++i) ok &= std::isfinite(p[i]);
-        return ok;
+        // An exponent of all ones: four vector instructions per load, against
+        // ten for isfinite's comparisons, whose time also varied with where
+        // the linker put the loop (four 224x224 images, host to host: 544 to
+        // 566 us, 536 so).
+        constexpr uint32_t kExponent = 0x7f800000u;
+        uint32_t bad = 0;
+        for (uint64_t i = a; i < b; ++i) {
+            uint32_t bits;
+            std::memcpy(&bits, p + i, 4);
+            bad |= (bits & kExponent) == kExponent;
+        }
+        return bad == 0;
     };
     constexpr uint64_t kChunk = 1ull << 20;
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());

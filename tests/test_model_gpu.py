@@ -266,6 +266,25 @@ def test_branches_are_bitwise_identical(models):
         m.set_branches(2)
 
 
+def test_only_finite_pixels_are_taken(models):
+    # Every bit pattern with an exponent of all ones is refused wherever it
+    # stands (the check runs over vectors, with a remainder); the largest
+    # finite values, subnormals and -0 are taken.
+    m = models(0, max_batch=8)
+    px = d.random_pixels(3, 1)
+    flat = px.reshape(-1)
+    keep = flat.copy()
+    for bits in (0x7F800000, 0xFF800000, 0x7F800001, 0x7FC00000, 0xFFFFFFFF):
+        for at in (0, 5, flat.size // 2 + 3, flat.size - 1):
+            flat[:] = keep
+            flat.view(np.uint32)[at] = bits
+            with pytest.raises(d.DINOv3Error, match="finite"):
+                m.forward(px)
+    flat[:] = keep
+    flat.view(np.uint32)[:4] = (0x7F7FFFFF, 0xFF7FFFFF, 0x00000001, 0x80000000)
+    assert m.forward(px).shape == (1, 201, 384)
+
+
 @pytest.mark.parametrize("images", [8, 23, 24, 31])
 def test_default_groups_on_both_sides_of_the_row_limit(weight_file, images):
     # A model whose grouping was never set: one group below 4800 rows (23
