@@ -10,8 +10,9 @@ issue order among themselves but are not ordered against register loads
 different results from launch to launch), so such a wait proves that an
 older stage has landed only if the N operations it lets stay in flight are
 all DMA loads: every step issues its register loads before its DMA loads.
-This test checks that rule on every barrier-ending wait with N > 0 of every
-kernel, in the code the compiler actually emitted (a reordering by the
+This test checks that rule on every wait with N > 0 that ends at a barrier or
+is written out in the source (attention_split_kernel waits for its Q fragments
+without a barrier) of every kernel, over its whole body, in the code the compiler actually emitted (a reordering by the
 compiler or by a later edit of the K loop would break it silently, showing
 only as rare run-to-run differences on the GPU). A negative control plants
 the mistake in a copy of the GEMM core (the step's DMA issued before its
@@ -28,18 +29,19 @@ import subprocess
 
 import pytest
 
+from test_kernel_arguments import build
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 KERNELS = os.path.join(ROOT, "dinov3-loom_amd", "csrc", "kernels")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-# The flags of dinov3-loom_amd/build.py for device code.
-FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang",
-         "-packed-fp32-ops", "--cuda-device-only", "-S"]
+FLAGS = [*build.COMMON, *build.DEVICE_FLAGS, "--cuda-device-only", "-S"]
 VMEM = re.compile(r"^(global_|buffer_|flat_|scratch_)")
 
 
 def assembly(src, out, include):
-    subprocess.check_call([HIPCC, *FLAGS, "-I", os.path.join(ROOT, "include"), "-I", include, src, "-o", out],
-                          stderr=subprocess.DEVNULL)
+    # Per kernel its instructions, those of an inline asm block between the
+    # marks "asm" and "end". A kernel may have several s_endpgm.
+    subprocess.check_call([HIPCC, *FLAGS, "-I", include, src, "-o", out], stderr=subprocess.DEVNULL)
     kernels, cur = {}, None
     for line in open(out):
         m = re.match(r"^(_Z\S+):", line)
@@ -48,11 +50,14 @@ def assembly(src, out, include):
             kernels[cur] = []
             continue
         s = line.strip()
-        if cur is None or not s or s.startswith((";", ".")):
-            continue
-        kernels[cur].append(s)
-        if s.startswith("s_endpgm"):
+        if s.startswith(".Lfunc_end"):
             cur = None
+        if cur is None or not s:
+            continue
+        if s.startswith((";;#ASMSTART", ";;#ASMEND")):
+            kernels[cur].append("asm" if "START" in s else "end")
+        elif not s.startswith((";", ".")):
+            kernels[cur].append(s)
     return kernels
 
 
@@ -61,25 +66,25 @@ def is_dma(ins):
 
 
 def violations(instructions):
-    """(checked waits, violations): for each `s_waitcnt vmcnt(N)` right
-    before an `s_barrier` with N > 0, the N vector-memory instructions
-    issued last before it must all be DMA loads."""
+    """(checked waits, violations): for each `s_waitcnt vmcnt(N)` with N > 0
+    right before an `s_barrier` or in an inline asm block, the N vector-memory
+    instructions issued last before it must all be DMA loads."""
     checked, bad = 0, []
     for i, ins in enumerate(instructions):
-        if not ins.startswith("s_barrier") or i == 0 or not instructions[i - 1].startswith("s_waitcnt"):
-            continue
-        m = re.search(r"vmcnt\((\d+)\)", instructions[i - 1])
+        m = re.search(r"vmcnt\((\d+)\)", ins) if ins.startswith("s_waitcnt") else None
         if not m or int(m.group(1)) == 0:
             continue
+        if not instructions[i + 1].startswith("s_barrier") and instructions[i - 1] != "asm":
+            continue
         n, tail = int(m.group(1)), []
-        for prev in reversed(instructions[:i - 1]):
+        for prev in reversed(instructions[:i]):
             if VMEM.match(prev):
                 tail.append(prev)
                 if len(tail) == n:
                     break
         checked += 1
         if len(tail) < n or not all(is_dma(t) for t in tail):
-            bad.append((instructions[i - 1], tail))
+            bad.append((ins, tail))
     return checked, bad
 
 
@@ -103,7 +108,8 @@ def test_every_k_loop_wait_counts_dma_only(hipcc, tmp_path):
             found[short] = checked
     print(found)
     for kernel in ("qkv_rope_kernel", "resid_kernel", "swiglu_kernel", "splitk_kernel", "attention_kernel",
-                   "attention_split_kernel"):
+                   "attention_split_kernel", "qkv_ring_kernel", "resid_ring_kernel", "swiglu_ring_kernel",
+                   "patch_ring_kernel", "attention_parallel_kernel"):
         assert any(k.startswith(kernel) and v > 0 for k, v in found.items()), kernel
 
 
@@ -136,6 +142,8 @@ def test_attention_kernels_touch_global_memory_only_as_designed(hipcc, tmp_path)
     # as DMA loads, the output as 16-byte buffer stores).
     kernels = assembly(os.path.join(KERNELS, "attention.hip"), str(tmp_path / "attention.s"), KERNELS)
     assert any("attention_split_kernel" in k for k in kernels)
+    # The wave-per-block kernels are read past their first exit.
+    assert any(sum(i.startswith("s_endpgm") for i in ins) > 1 for k, ins in kernels.items() if "parallel" in k)
     for name, ins in kernels.items():
         for i in ins:
             op = i.split()[0]
