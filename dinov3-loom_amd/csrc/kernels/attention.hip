@@ -431,7 +431,7 @@ __global__ __launch_bounds__(kThreads, 3) void attention_kernel(DHX_ATTENTION_PA
 // tokens 5.1 -> 4.2 us to 6 images, 69 tokens 4.25 -> 3.0, 261 tokens 6.5 ->
 // 5.2, 405 tokens 8.0 -> 6.4; what is left is the launch, the loads, one
 // softmax step and the 2 N MFMAs of a PV chain.
-constexpr int kMaxParallel = 15;
+constexpr int kMaxParallel = 14;  // 446 tokens; the next square grid's 489 take 16 blocks
 
 template <int N>
 struct ParallelLds {
@@ -714,7 +714,7 @@ hipError_t launch_split(const AttentionArgs& a, int groups, hipStream_t s) {
 
 }  // namespace
 
-// To 480 tokens, where one round of 32-query workgroups covers the launch, one
+// To 446 tokens, where one round of 32-query workgroups covers the launch, one
 // wave per key block (whole forward, against the walks below: 224x224 batch 1
 // 304 -> 294 us, batch 6 332 -> 322, 128x128 batch 4 302 -> 286, 256x256 batch
 // 4 351 -> 334, 320x320 batch 3 368 -> 349; in two rounds 224x224 batch 8 351

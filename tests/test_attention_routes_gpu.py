@@ -35,12 +35,14 @@ def inputs(grid, images, scale=2.0):
     return [f16(rng.normal(size=(rows, 384)) * s) for s in (scale, 1.0, 1.0)]
 
 
-# (grid, images of the large launch, images of the others): 1, 3, 5, 7, 8, 9
-# and 14 key blocks (a wave per block up to 256 workgroups of 32 queries), 16
-# and 19 blocks (64-query workgroups up to 256 of them), 1029 tokens (64
-# queries to 2 images, 128 from 3, the unrolled walk from 5), 2030 tokens.
-ROUTES = [(4, 50, (1, 42, 43)), (8, 20, (1, 14, 15)), (12, 12, (1, 8, 9)), (14, 10, (1, 6, 7)), (15, 8, (1, 5, 6)),
-          (16, 8, (1, 4, 5)), (21, 6, (1, 3, 4)), (22, 8, (1, 4, 5, 6)), (24, 8, (1, 4, 5)), (32, 6, (1, 2, 3, 4, 5)),
+# (grid, images of the large launch, images of the others): 1 to 14 key blocks
+# (a wave per block up to 256 workgroups of 32 queries), 16 and 19 blocks
+# (64-query workgroups up to 256 of them, 192 beside another launch), 1029
+# tokens (64 queries to 2 images, 128 from 3, the unrolled walk from 5 and
+# beside another launch), 2030 tokens.
+ROUTES = [(4, 50, (1, 42, 43)), (7, 24, (1, 21, 22)), (8, 20, (1, 14, 15)), (10, 14, (1, 10, 11)), (12, 12, (1, 8, 9)),
+          (13, 10, (1, 7, 8)), (14, 10, (1, 6, 7)), (15, 8, (1, 5, 6)), (16, 8, (1, 4, 5)), (17, 6, (1, 4, 5)),
+          (18, 5, (1, 3, 4)), (19, 5, (1, 3, 4)), (20, 5, (1, 3, 4)), (21, 6, (1, 3, 4)), (22, 8, (1, 4, 5, 6)), (24, 8, (1, 4, 5)), (32, 6, (1, 2, 3, 4, 5)),
           (45, 3, (1, 2))]
 
 
