@@ -34,12 +34,9 @@ void parallel_copy(void* dst, const void* src, uint64_t n) noexcept {
     for (auto& th : pool) th.join();
 }
 
-Copier::Copier(bool threaded) {
-    if (threaded) worker_ = std::thread([this] { run(); });
-}
+Copier::Copier() { worker_ = std::thread([this] { run(); }); }
 
 Copier::~Copier() {
-    if (!worker_.joinable()) return;
     {
         std::lock_guard<std::mutex> lock(m_);
         stop_ = true;
@@ -50,11 +47,6 @@ Copier::~Copier() {
 
 uint64_t Copier::submit(void* dst, const void* src, uint64_t n) {
     std::lock_guard<std::mutex> lock(m_);
-    if (!worker_.joinable()) {
-        parallel_copy(dst, src, n);
-        ++done_;
-        return submitted_++;
-    }
     jobs_.push_back(Job{dst, src, n});
     work_.notify_all();
     return submitted_++;

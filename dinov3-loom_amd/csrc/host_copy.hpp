@@ -22,9 +22,7 @@ void parallel_copy(void* dst, const void* src, uint64_t n) noexcept;
 // thread that launches keeps every HIP call and hands the copies over.
 class Copier {
 public:
-    // threaded = false: submit() copies at once on the calling thread (one
-    // chunk has nothing to overlap, and a thread would only add its start).
-    explicit Copier(bool threaded);
+    Copier();
     // Runs every queued copy before returning: their buffers outlive the
     // caller's scope, also when the caller is unwinding an exception.
     ~Copier();
@@ -48,7 +46,7 @@ private:
     std::deque<Job> jobs_;
     uint64_t submitted_ = 0, done_ = 0;
     bool stop_ = false;
-    std::thread worker_;  // started (if threaded) in the constructor's body, once the members above exist
+    std::thread worker_;  // started in the constructor's body, once the members above exist
 };
 
 }  // namespace dhx

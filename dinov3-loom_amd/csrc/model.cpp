@@ -286,7 +286,7 @@ public:
             return;
         }
         std::vector<uint64_t> filled(chunks), drained(chunks);
-        Copier copier(true);
+        Copier copier;
         // Chunk i's pixels into slot i % 2's input staging, once the slot's
         // previous upload has left it.
         auto fill = [&](uint64_t i) {

@@ -52,7 +52,7 @@ void check_parallel_copy(std::mt19937_64& rng) {
 // each destination right after waiting for its ticket (the pattern of the
 // forward pipeline), and chained copies (a -> b, then b -> c) prove that
 // copies run in submission order.
-void check_copier(std::mt19937_64& rng, bool threaded) {
+void check_copier(std::mt19937_64& rng) {
     const int jobs = 96;
     std::vector<std::vector<unsigned char>> src(jobs), mid(jobs), dst(jobs);
     for (int i = 0; i < jobs; ++i) {
@@ -61,7 +61,7 @@ void check_copier(std::mt19937_64& rng, bool threaded) {
         mid[i].assign(n, 0);
         dst[i].assign(n, 0);
     }
-    dhx::Copier copier(threaded);
+    dhx::Copier copier;
     std::vector<uint64_t> first(jobs), second(jobs);
     for (int i = 0; i < jobs; ++i) {
         first[i] = copier.submit(mid[i].data(), src[i].data(), src[i].size());
@@ -85,7 +85,7 @@ void check_drain_on_destruction(std::mt19937_64& rng) {
         dst[i].assign(src[i].size(), 0);
     }
     {
-        dhx::Copier copier(true);
+        dhx::Copier copier;
         for (int i = 0; i < jobs; ++i) copier.submit(dst[i].data(), src[i].data(), src[i].size());
     }
     for (int i = 0; i < jobs; ++i) expect(dst[i] == src[i], "queued copy ran before destruction", (uint64_t)i);
@@ -96,8 +96,8 @@ void check_drain_on_destruction(std::mt19937_64& rng) {
 int main() {
     std::mt19937_64 rng(20261202);
     check_parallel_copy(rng);
-    check_copier(rng, true);
-    check_copier(rng, false);
+    check_copier(rng);
+    check_copier(rng);
     check_drain_on_destruction(rng);
     std::printf("ok %d\n", g_checks);
     return 0;
