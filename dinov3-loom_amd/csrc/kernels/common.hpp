@@ -178,21 +178,38 @@ struct RowNorm {
     float mean, rstd;
 };
 
-// From a row's 12 statistics floats, loaded as three float4 (a, b, c).
-__device__ __forceinline__ RowNorm row_norm(float4_t a, float4_t b, float4_t c) {
-    const float mk[6] = {a[0], a[2], b[0], b[2], c[0], c[2]};
-    const float m2 = (a[1] + a[3]) + (b[1] + b[3]) + (c[1] + c[3]);
-    const float mean = (((mk[0] + mk[1]) + (mk[2] + mk[3])) + (mk[4] + mk[5])) * (1.0f / 6.0f);
-    float dev = 0.f;
+// d[0]^2 + ... + d[N - 1]^2: d[1]^2 rounded, the others fused onto it in order.
+template <int N>
+__device__ __forceinline__ float sum_of_squares(const float (&d)[N]) {
+    float q = d[1] * d[1];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) dev += (mk[i] - mean) * (mk[i] - mean);
-    const float var = (m2 + 64.0f * dev) * (1.0f / kHidden);
-    return RowNorm{mean, rsqrtf(var + 1e-5f)};
+    for (int i = 0; i < N; ++i)
+        if (i != 1) q = fmaf(d[i], d[i], q);
+    return q;
 }
 
+// From a row's 12 statistics floats, loaded as three float4 (a, b, c).
+// Its FMAs are written out, as are those of the epilogues: contracted by the
+// compiler, each kernel's own way, two tile shapes could differ in the last
+// bit. FUSED: a slot's deviation from the mean as one FMA on the sum (the QKV
+// kernels), else a difference (the SwiGLU kernels).
+template <bool FUSED>
+__device__ __forceinline__ RowNorm row_norm(float4_t a, float4_t b, float4_t c) {
+#pragma clang fp contract(off)
+    const float mk[6] = {a[0], a[2], b[0], b[2], c[0], c[2]};
+    const float m2 = (a[1] + a[3]) + (b[1] + b[3]) + (c[1] + c[3]);
+    const float sum = ((mk[0] + mk[1]) + (mk[2] + mk[3])) + (mk[4] + mk[5]), mean = sum * (1.0f / 6.0f);
+    float d[6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) d[i] = FUSED ? fmaf(sum, -1.0f / 6.0f, mk[i]) : mk[i] - mean;
+    const float dev = sum_of_squares(d);
+    return RowNorm{mean, rsqrtf(fmaf(fmaf(64.0f, dev, m2), 1.0f / kHidden, 1e-5f))};
+}
+
+template <bool FUSED>
 __device__ __forceinline__ RowNorm row_norm(const float* stats, size_t row) {
     const float4_t* p = (const float4_t*)(stats + row * 12);
-    return row_norm(p[0], p[1], p[2]);
+    return row_norm<FUSED>(p[0], p[1], p[2]);
 }
 
 }  // namespace dhx

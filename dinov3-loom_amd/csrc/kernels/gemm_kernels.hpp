@@ -62,10 +62,10 @@ __device__ __forceinline__ void pair_stats(float* stats, size_t m, int slot, con
     for (int e = 0; e < 32; ++e) s += v[e];
     s = half_pair_sum(s);
     const float mean = s * (1.0f / 64.0f);
-    float q = 0.f;
+    float d[32];
 #pragma unroll
-    for (int e = 0; e < 32; ++e) q += (v[e] - mean) * (v[e] - mean);
-    q = half_pair_sum(q);
+    for (int e = 0; e < 32; ++e) d[e] = v[e] - mean;
+    const float q = half_pair_sum(sum_of_squares(d));
     if (store && hi == 0) *(float2_t*)(stats + m * kStatFloats + slot * 2) = float2_t{mean, q};
 }
 
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
                 const int lane = tid & 63, r0 = (tid >> 6) % T::WGM * T::TM;
 #pragma unroll
                 for (int j = 0; j < T::FM; ++j) {
-                    const RowNorm rn = row_norm(raw[j][0], raw[j][1], raw[j][2]);
+                    const RowNorm rn = row_norm<true>(raw[j][0], raw[j][1], raw[j][2]);
                     if (lane < 32) rows_norm[r0 + j * 32 + lane] = float2_t{rn.mean, rn.rstd};
                 }
             }
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void qkv_rin
     gemm_main_ring<T, NST, kHidden / T::BK>(ring, bufs, acc, [&](Acc<T>&, auto S) {
         if constexpr (LN && decltype(S)::value == 0) {
 #pragma unroll
-            for (int j = 0; j < T::FM; ++j) rn[j] = row_norm(stats, f.row(j) - m0);
+            for (int j = 0; j < T::FM; ++j) rn[j] = row_norm<true>(stats, f.row(j) - m0);
         }
     });
     qkv_epilogue<T, LN>(p, acc, f, m0, n0, bias, wsum, rope_lds,
@@ -548,7 +548,8 @@ __device__ __forceinline__ void resid_epilogue(const ResidArgs& p, const Acc<T>&
             for (int g = 0; g < 4; ++g) {
                 const int nt = f.col(i, g) - n0;  // column in the tile
                 const float4_t bl = *(const float4_t*)&cst[0][nt], l = *(const float4_t*)&cst[1][nt];
-                u[g] = group4(acc.v[i][j], g) * l + bl;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) u[g][e] = fmaf(acc.v[i][j][4 * g + e], l[e], bl[e]);
             }
             frag_swap(u[0], u[1]);
             frag_swap(u[2], u[3]);
@@ -703,11 +704,13 @@ __device__ __forceinline__ void swiglu_epilogue(const SwigluArgs& p, const Acc<T
             for (int g = 0; g < 4; ++g) {
                 const int c = g * 8 + f.hi * 4, nl = f.n_base - n0 + 64 * q + c;
                 float4_t gate = group4(acc.v[2 * q][j], g), up = group4(acc.v[2 * q + 1][j], g);
-                const float4_t gs = gate * sg + *(const float4_t*)&bias[nl];
-                const float4_t us = up * su + *(const float4_t*)&bias[nl + 32];
+                const float4_t bg = *(const float4_t*)&bias[nl], bu = *(const float4_t*)&bias[nl + 32];
                 float4_t r;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) r[e] = gs[e] * us[e] * fast_rcp(1.0f + fast_exp2(gs[e]));
+                for (int e = 0; e < 4; ++e) {
+                    const float gs = fmaf(gate[e], sg, bg[e]), us = fmaf(up[e], su, bu[e]);
+                    r[e] = gs * us * fast_rcp(1.0f + fast_exp2(gs));
+                }
                 y[g] = to_half4(r);
             }
 #pragma unroll
@@ -785,7 +788,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? 3 : 2) void swiglu_kernel(
                 cst[1][tid] = cw;
             }
 #pragma unroll
-            for (int j = 0; j < T::FM; ++j) rn[j] = LN ? row_norm(raw[j][0], raw[j][1], raw[j][2]) : RowNorm{0.f, 1.f};
+            for (int j = 0; j < T::FM; ++j) rn[j] = LN ? row_norm<false>(raw[j][0], raw[j][1], raw[j][2]) : RowNorm{0.f, 1.f};
         },
         [&](const Acc<T>& acc, int m0, int n0) {
         const Frag<T> f(m0, n0);
@@ -840,7 +843,7 @@ __global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void swiglu_
         if constexpr (s == 0) {
             if (tid < T::BN) bias[tid] = raw[tid] * swiglu_scale(tid);
 #pragma unroll
-            for (int j = 0; j < T::FM; ++j) rn[j] = LN ? row_norm(stats, f.row(j) - m0) : RowNorm{0.f, 1.f};
+            for (int j = 0; j < T::FM; ++j) rn[j] = LN ? row_norm<false>(stats, f.row(j) - m0) : RowNorm{0.f, 1.f};
         }
         if constexpr (LN && s > 0 && s * T::BK % 64 == 0 && s * T::BK <= 256) {
             static_for<T::FN>([&](auto I) {
