@@ -647,21 +647,23 @@ def test_stats_producer_adversarial_rows(eng):
 
 
 # ---------------------------------------------------------------------------
-# Bitwise repeatability of the DMA-fed kernels at the shapes the bench runs:
-# batch 64 and 32 at 224x224 and batch 8 at 512x512. The GEMMs move their
-# weight stages, and attention its K/V blocks, into LDS with DMA loads;
+# Bitwise repeatability of the DMA-fed kernels at the shapes the bench runs,
+# batch 64 and 32 at 224x224 and batch 8 at 512x512, and at one size inside the
+# range of every ring of the small launches (201, 1005, 1608, 2412 and 4020
+# rows). The GEMMs move their weight stages (the rings both operands), and attention its K/V blocks, into LDS with DMA loads;
 # waiting for one correctly depends on the order in which those loads and
 # the register loads complete, and a wrong wait shows up as results that
 # change from launch to launch (stale data in LDS), not as a fault.
 
 SHAPES = {"b64": (64, 14), "b32": (32, 14), "512b8": (8, 32)}
+GEMM_SHAPES = {**SHAPES, "b1": (1, 14), "b5": (5, 14), "b8": (8, 14), "b12": (12, 14), "b20": (20, 14)}
 
 
-@pytest.mark.parametrize("shape", list(SHAPES))
+@pytest.mark.parametrize("shape", list(GEMM_SHAPES))
 @pytest.mark.parametrize("kernel", ["qkv_ln", "swiglu_ln", "resid_384", "resid_1536", "splitk"])
 def test_gemm_bitwise_repeatable(eng, kernel, shape):
     rng = np.random.default_rng(5)
-    images, grid = SHAPES[shape]
+    images, grid = GEMM_SHAPES[shape]
     T = grid * grid + 5
     tpad = (T + 127) // 128 * 128
     M = images * T
@@ -711,16 +713,37 @@ def test_gemm_bitwise_repeatable(eng, kernel, shape):
         assert np.array_equal(first, again), f"{kernel}: launch {rep + 2} differs in {int((first != again).sum())} elements"
 
 
-ATTN_SHAPES = {**SHAPES, "384b8": (8, 24)}
+@pytest.mark.parametrize("images", [1, 6, 16])
+def test_patch_embedding_bitwise_repeatable(eng, images):
+    # 196 and 1176 patches run patch_ring_kernel, 3136 the tiles without DMA.
+    rng = np.random.default_rng(images)
+    px = up(eng, rng.normal(size=(images, 3, 224, 224)).astype(np.float32))
+    w = up(eng, f16(rng.normal(size=(384, 768)) * 0.02))
+    b, prefix, pstats = (up(eng, rng.normal(size=s).astype(np.float32)) for s in ((384,), (5, 384), (5, 12)))
+
+    def once():
+        x, st = allocf(eng, images * 201, 384), eng.allocate(images * 201 * 48)
+        run(eng, K_PATCH_S, [images, 14], [px, w, b, prefix, pstats, x, st])
+        return np.concatenate([readf(eng, x, images * 201, 384).astype(np.float32).ravel(),
+                               eng.read(st, np.float32, (images * 201 * 12,))])
+
+    first = once()
+    for rep in range(4):
+        assert np.array_equal(first, once()), f"launch {rep + 2}"
 
 
-@pytest.mark.parametrize("shape", ["b64", "512b8", "384b8"])
+ATTN_SHAPES = {**SHAPES, "384b8": (8, 24), "b1": (1, 14), "512b1": (1, 32), "256b16": (16, 16)}
+
+
+@pytest.mark.parametrize("shape", ["b64", "512b8", "384b8", "b1", "512b1", "256b16"])
 def test_attention_bitwise_repeatable(eng, shape):
-    # T = 201 runs attention_kernel<7> (seven 32-key blocks, unrolled),
-    # T = 1029 attention_split_kernel<17> (two key halves of 17 unrolled
-    # 32-key blocks), T = 581 (384x384) attention_kernel<0>, the run-time
-    # count of 64-key blocks that serves every other image size; all three
-    # DMA K/V two blocks ahead into three buffers.
+    # 224x224: attention_kernel<7> (seven 32-key blocks, unrolled) at batch 64,
+    # attention_parallel_kernel<7> (a wave per block) at batch 1; 512x512:
+    # attention_split_kernel<17, 4> (two key halves of 17 unrolled 32-key
+    # blocks) at batch 8, <0, 2> (64 queries, run-time count) at batch 1;
+    # 384x384 batch 8: <0, 4>; 256x256 batch 16: attention_kernel<0>, the
+    # run-time count of 64-key blocks. All but the parallel kernel DMA K/V two
+    # blocks ahead into three buffers.
     images, grid = ATTN_SHAPES[shape]
     rng = np.random.default_rng(12)
     T = grid * grid + 5

@@ -28,8 +28,10 @@ def _threads(gpu):
 def models(weight_file):
     cache = {}
 
-    def get(preset=0, max_batch=4, image_size=224):
-        key = (preset, max_batch, image_size)
+    # grouped: a model apart, for the tests that set its image groups (there is
+    # no way back to the choice by size).
+    def get(preset=0, max_batch=4, image_size=224, grouped=False):
+        key = (preset, max_batch, image_size, grouped)
         if key not in cache:
             cache[key] = d.DINOv3.load(weight_file(preset), d.Options(0, max_batch, image_size))
         return cache[key]
@@ -159,19 +161,17 @@ def test_batch_64_stress_every_grouping(models, oracle_weights):
     # of three image groups (and the last image) against the
     # oracle; all 64 outputs bitwise equal for every grouping bench.py may
     # pick (1-4 concurrent groups) and to the same images run as batches of 16.
-    m = models(1, max_batch=64)
+    m = models(1, max_batch=64, grouped=True)
     px = d.random_pixels(22, 64)
     m.set_branches(3)
     out = m.forward(px)
     assert out.shape == (64, 201, 384) and np.all(np.isfinite(out))
     for i in (0, 21, 42, 63):
         compare(out[i], oracle.forward(oracle_weights(1), px[i], 14), f"b64 stress image {i}", 1)
-    try:
-        for n in (1, 2, 4):
-            m.set_branches(n)
-            assert np.array_equal(m.forward(px), out), f"{n} groups"
-    finally:
-        m.set_branches(2)
+    for n in (1, 2, 4):
+        m.set_branches(n)
+        assert np.array_equal(m.forward(px), out), f"{n} groups"
+    m = models(1, max_batch=64)
     for first in range(0, 64, 16):
         assert np.array_equal(m.forward(px[first:first + 16]), out[first:first + 16]), first
 
@@ -182,17 +182,14 @@ def test_512_batch_8_grouped_plan(models, oracle_weights):
     # the batch bitwise equal to one group, to batches of 2 and, for those
     # two images, to batches of 1 (the default plan uses the residual GEMM
     # at every batch size, so an image's bits do not depend on the batch).
-    m = models(1, max_batch=8, image_size=512)
+    m = models(1, max_batch=8, image_size=512, grouped=True)
     px = d.random_pixels(23, 8, 512)
     out = m.forward(px)
     assert out.shape == (8, 1029, 384) and np.all(np.isfinite(out))
     for i in (0, 7):
         compare(out[i], oracle.forward(oracle_weights(1), px[i], 32), f"512 b8 image {i}", 1)
-    try:
-        m.set_branches(1)
-        assert np.array_equal(m.forward(px), out)
-    finally:
-        m.set_branches(2)
+    m.set_branches(1)
+    assert np.array_equal(m.forward(px), out)
     assert np.array_equal(m.forward(px[:2]), out[:2])
     assert np.array_equal(m.forward(px[6:]), out[6:])
     assert np.array_equal(m.forward(px[:1]), out[:1])
@@ -248,22 +245,20 @@ def test_branches_are_bitwise_identical(models):
     # Image groups recorded as concurrent graph branches: every grouping gives
     # the same bits (a row's arithmetic never depends on its group), in both
     # graph replay and the direct-dispatch path used by benchmark().
-    m = models(1, max_batch=16)
+    m = models(1, max_batch=16, grouped=True)
     px = d.random_pixels(8, 16)
     m.set_branches(1)
-    try:
-        base = m.forward(px)
-        for n in (2, 3, 4):
-            m.set_branches(n)
-            assert np.array_equal(m.forward(px), base), f"{n} branches"
-            assert np.array_equal(m.forward(px[:9]), base[:9]), f"{n} branches, 9 images"
-        t = m.benchmark(px, 10)
-        assert t.samples == 10
-        assert np.array_equal(m.forward(px), base)
+    base = m.forward(px)
+    for n in (2, 3, 4):
+        m.set_branches(n)
+        assert np.array_equal(m.forward(px), base), f"{n} branches"
+        assert np.array_equal(m.forward(px[:9]), base[:9]), f"{n} branches, 9 images"
+    t = m.benchmark(px, 10)
+    assert t.samples == 10
+    assert np.array_equal(m.forward(px), base)
+    for n in (0, 5):
         with pytest.raises(d.DINOv3Error, match="branches must be 1..4"):
-            m.set_branches(5)
-    finally:
-        m.set_branches(2)
+            m.set_branches(n)
 
 
 def test_only_finite_pixels_are_taken(models):
@@ -333,9 +328,10 @@ def test_512_high_resolution(models, oracle_weights, preset):
 @pytest.mark.parametrize("size", [16, 64, 256, 384])
 def test_other_image_sizes(models, oracle_weights, size):
     # Image sizes other than 224 and 512 (any multiple of 16 is accepted):
-    # 6 (the smallest: one patch), 21, 261 and 581 tokens run the attention
-    # kernel with a run-time count of 64-key blocks, and the RoPE tables and
-    # patch gather of 1x1, 4x4, 16x16 and 24x24 grids. Stress preset against the oracle; each image of the
+    # 6 (the smallest: one patch), 21 and 261 tokens run the attention kernel
+    # with a wave per key block, 581 the one with two key halves on 64-query
+    # workgroups, and the RoPE tables and patch gather are those of 1x1, 4x4,
+    # 16x16 and 24x24 grids. Stress preset against the oracle; each image of the
     # batch of two equals it alone, bitwise.
     G = size // 16
     m = models(1, max_batch=2, image_size=size)
