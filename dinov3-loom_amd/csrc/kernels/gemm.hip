@@ -8,20 +8,21 @@ namespace {
 using gemm::Tile;
 using gemm::tiles_for;
 
-// The patch embedding stages both operands in LDS (its A operand is gathered
-// from pixels); the others take activations in fragment order straight into
-// registers, waves stacked along M. The residual GEMMs (N = 384: too few
-// 128x128 tiles to fill 256 CUs) use 128x64 tiles, twice as many workgroups
-// of a quarter of the registers.
+// Tiles of the launches of several rounds of workgroups (the rings' follow
+// below). The patch embedding stages both operands in LDS (its A operand is
+// gathered from pixels); the others take activations in fragment order
+// straight into registers, waves stacked along M. The residual GEMMs (N = 384:
+// too few 128x128 tiles to fill 256 CUs) use 128x64 tiles, twice as many
+// workgroups of a quarter of the registers.
 using PatchTile = Tile<64, 128, 2, 2>;
 // QKV on 32-deep stages (24 KB of weight buffers; its RoPE angles wait in
 // LDS, not registers): four workgroups per CU, so a batch of 64 (909 tiles)
 // runs as one round of workgroups.
 using QkvTile = Tile<128, 128, 4, 1, 32>;
-// QKV for launches of fewer rows (512x512 batch 8's image groups): 128x64
-// tiles (one head per wave), twice the
-// workgroups. Same stage depth, and the LayerNorm fold is applied in the
-// epilogue, so a row's result is bitwise the same on either shape.
+// QKV for launches of fewer rows (the image groups of batch 32 and of 512x512
+// batch 8): 128x64 tiles (one head per wave), twice the workgroups. Same stage
+// depth, and the LayerNorm fold is applied in the epilogue, so a row's result
+// is bitwise the same on either shape.
 using QkvTileS = Tile<128, 64, 4, 1, 32>;
 constexpr int kQkvSmallRows = 5120;
 using ResidTile = Tile<128, 64, 4, 1>;
@@ -136,12 +137,13 @@ hipError_t launch_resid(const ResidArgs& a, hipStream_t s) {
     // 8.5 us off each of these (201 rows 295.3 -> 286.8, 1005 rows 315.6 ->
     // 308.5; three or four 128-deep stages 294, 293, 1608 rows 355 -> 377).
     // Beside another image group's kernels (a.shared) the 128x64 ring, which
-    // takes a CU's LDS whole, loses to the tiles below (705 -> 742 us at 2 x
-    // 3216 rows).
+    // takes a CU's LDS whole, loses to the tiles below (620 -> 629 us at 2 x
+    // 2814 rows, 667 -> 728 at 2 x 3216).
     // One more size for the down projection, 128x128 tiles to 10880 rows: 6432
     // rows 736 -> 699 us, 8643 rows 886 -> 858, 8232 rows 1029 -> 1008 (one
-    // chain); beside another group 705 -> 733 at 2 x 6432 rows. The o-projection,
-    // with three stages to a tile, gains nothing from it.
+    // chain); beside another group 1003 -> 992 at 2 x 5427 rows, 1100 -> 1105 at
+    // 2 x 6432. The o-projection, with three stages to a tile, gains nothing
+    // from it.
     const int round = a.rows <= kRound / 6 * 32   ? 32
                       : a.rows <= kRound / 6 * 64 ? 64
                       : a.shared                  ? 0

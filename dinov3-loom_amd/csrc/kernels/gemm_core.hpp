@@ -2,8 +2,8 @@
 // accumulation, shared by every GEMM variant of the forward pass.
 //
 // A workgroup of WGM x WGN waves owns a BM x BN output tile; the K loop walks
-// BK-deep stages. Two loops:
-// - gemm_main (the patch embedding): both operands HBM/L2 -> registers ->
+// BK-deep stages. Three loops:
+// - gemm_main (the patch embedding's tiles): both operands HBM/L2 -> registers ->
 //   LDS (row pitch LDK) with two register sets and two LDS buffers, so the
 //   loads of stage s+2 are in flight while stage s feeds the MFMAs and stage
 //   s+1 is written to LDS.
@@ -11,7 +11,9 @@
 //   order straight into registers (ActFrags), weights in fragment order moved
 //   into three LDS buffers by DMA (WeightDma); its comment has the ordering
 //   rules the waits rely on.
-// The barriers only wait for LDS traffic (and, in the DMA loop, for the DMA
+// - gemm_main_ring (QKV, residual, SwiGLU in launches of one round of
+//   workgroups): both operands moved by DMA into a ring of LDS stages (Ring).
+// The barriers only wait for LDS traffic (and, in the DMA loops, for the DMA
 // loads they must): __syncthreads() would also drain every outstanding
 // global load (its workgroup release fence waits on vmcnt(0)) and serialise
 // the pipeline. Loads are unconditional where possible (indices clamped) so

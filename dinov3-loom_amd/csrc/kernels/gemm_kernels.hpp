@@ -5,10 +5,11 @@
 // matmul_qkv_rope_f16_wmma.loom, matmul_resid_f16_wmma.loom,
 // matmul_swiglu_f16_wmma.loom and matmul_splitk_f16_wmma.loom.
 //
-// Activations (x, h, attn, act) are kept in fragment order (common.hpp):
-// every GEMM except the patch embedding loads its activation operand
-// straight into registers (ActFrags) and stages only the weights in LDS,
-// with the workgroup's waves stacked along M (32 x 128 per wave).
+// Activations (x, h, attn, act) are kept in fragment order (common.hpp). The
+// GEMMs of several rounds of workgroups load them straight into registers
+// (ActFrags) and stage only the weights in LDS, with the workgroup's waves
+// stacked along M; the rings of the small launches (*_ring_kernel) move both
+// operands through LDS, and the patch embedding gathers its own from pixels.
 #pragma once
 #include "gemm_core.hpp"
 #include "launch.hpp"
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
     const QkvArgs p{h_, w_, bias_, cos_, sin_, q_, k_, v_, images_, grid_, tpad_, stats_, wsum_};
     static_assert(T::TN % kHeadDim == 0 && kHidden % T::BN == 0 && T::WGN == 1,
                   "whole heads per wave and tile, whole rows per wave");
-        __shared__ __attribute__((aligned(16))) half_t wb0[T::WF_HALFS], wb1[T::WF_HALFS], wb2[T::WF_HALFS];
+    __shared__ __attribute__((aligned(16))) half_t wb0[T::WF_HALFS], wb1[T::WF_HALFS], wb2[T::WF_HALFS];
     __shared__ __attribute__((aligned(16))) float cst[2][T::BN];  // bias, wsum of the tile's columns
     __shared__ float2_t rows_norm[T::BM];                          // (mean, rstd) of the tile's rows
     extern __shared__ __attribute__((aligned(16))) float rope_lds[];  // rope_table_dma's four tables
@@ -472,8 +473,8 @@ __global__ __launch_bounds__(T::THREADS, T::FM == 1 ? (T::BK == 32 ? 4 : 3) : 2)
 // the launcher and resid_ring_kernel): everything the epilogue needs comes
 // through LDS by DMA ahead of the stages. In a forward the launch starts with
 // cold L2s, and qkv_rope_kernel's twelve 32-deep steps then each wait for a
-// load; here up to four 64-deep stages are in flight. At 201 rows 5.1 -> 4.7
-// us alone with warm caches, 2.3 us per launch less in the forward.
+// load; here three 64-deep stages are in flight (two on 128-row tiles). At 201
+// rows 5.1 -> 4.7 us alone with warm caches, 2.3 us per launch less in the forward.
 template <class T, int NST, bool LN>
 __global__ __launch_bounds__(T::THREADS, (Ring<T, NST>::MIN_WAVES)) void qkv_ring_kernel(DHX_QKV_PARAMS) {
     const QkvArgs p{h_, w_, bias_, cos_, sin_, q_, k_, v_, images_, grid_, tpad_, stats_, wsum_};

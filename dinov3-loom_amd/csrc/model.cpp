@@ -40,10 +40,13 @@ constexpr uint64_t kMinBranchImages = 4;
 // chains of half the rows fill each other's partial rounds of workgroups; but
 // below this the tiles chosen by size fit a whole launch in about one round,
 // and the second chain only takes compute units from the first. Replays of
-// one group | two, us: 224x224 8 images (1608 rows) 354 | 499, 16 (3216)
-// 459 | 497, 20 (4020) 483 | 545, 24 (4824) 564 | 559, 28 (5628) 675 | 619,
-// 64 (12864) 1167 | 1092; 384x384 8 images (4648 rows) 611 | 687, 10 (5810)
-// 783 | 755; 64x64 64 images (1344 rows) 341 | 442.
+// one group | two, us: 224x224 8 images (1608 rows) 354 | 453, 16 (3216)
+// 459 | 501, 20 (4020) 485 | 557, 23 (4623) 548 | 580, 24 (4824) 552 | 575 and
+// on another card 598 | 583, 28 (5628) 671 | 644, 32 (6432) 706 | 674, 40
+// (8040) 769 | 758, 43 (8643) 876 | 828, 48 (9648) 930 | 897, 56 (11256)
+// 1128 | 1038, 64 (12864) 1168 | 1105; 384x384 8 images (4648 rows) 600 | 662,
+// 9 (5229) 742 | 720, 10 (5810) 773 | 765; 512x512 8 (8232) 1044 | 975;
+// 1024x1024 8 (32808) 5860 | 5436; 64x64 64 images (1344 rows) 340 | 450.
 constexpr uint64_t kTwoGroupRows = 4800;
 
 // hub.rs:7-11
